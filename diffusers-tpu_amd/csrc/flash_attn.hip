@@ -10,7 +10,10 @@
 // Decomposition
 //   * One workgroup = 8 wavefronts = 256 query rows of one (batch, head);
 //     wavefront w owns rows 32w .. 32w+31 for the whole key sweep.  Waves w
-//     and w+4 share a SIMD.
+//     and w+4 share a SIMD.  Few query blocks or few tiles run in smaller
+//     row blocks (row_shape): 128 rows of 4 wavefronts, two workgroups per
+//     CU, or row wavefronts times key groups.  These keep rings of 2 stages
+//     (K two tiles ahead, V one) and are otherwise the same.
 //   * Keys/values stream through LDS in 64-key tiles, a ring of 4 (K, V)
 //     stages (128 KiB: the four K tiles, then the four V tiles).  Tile t is
 //     requested two iterations before its QK step with
@@ -77,17 +80,14 @@
 namespace dt {
 namespace {
 
-constexpr int kNW = 8;               // wavefronts per workgroup
-constexpr int kBQ = kNW * 32;        // query rows per workgroup
 constexpr int kBKV = 64;             // keys per tile
-constexpr int kNStage = 4;           // LDS ring depth
+constexpr int kBQ = 256;             // query rows of a workgroup of 8 wavefronts
 // Tiles requested ahead of their use.  Two: three kept a third tile per CU
 // in flight and measured 0.2-0.7 % slower with bf16 keys (V7, V4, I1, I2,
 // two boxes) and 3.3 % slower with E4M3 keys at V7, the deeper DMA queue
 // lengthening every tile's latency; with two, one stage of the ring is
 // always idle.
 constexpr int kDist = 2;
-constexpr int kRowsPerWave = kBKV / kNW;  // tile rows each wave loads
 
 // LDS layout for head dim D: the K tiles of the 4 ring stages (bf16: 2D-byte
 // rows; E4M3: D-byte rows), then the 4 V tiles (2D-byte key rows, or with
@@ -96,17 +96,21 @@ constexpr int kRowsPerWave = kBKV / kNW;  // tile rows each wave loads
 // is unrolled over the ring, so the stage is a constant), which the LDS
 // read encodes as its immediate offset: no per-tile address arithmetic.
 // QK8 selects E4M3 keys (the reference's qk_fp8).
-template <int D, bool QK8>
+// A workgroup is R row wavefronts (32 query rows each) times G key groups,
+// each group with a ring of its own.
+template <int D, bool QK8, int R>
 struct Stage {
+  static constexpr int kNStage = R == 8 ? 4 : 2;     // LDS ring depth
+  static constexpr int kRowsPerWave = kBKV / R;      // tile rows each wave loads
   static constexpr int kKRow = QK8 ? D : 2 * D;  // bytes of a K row
   static constexpr int kVRow = 2 * D;            // bytes of a V key row
   static constexpr int kKTileB = kBKV * kKRow;
   static constexpr int kVTileB = kBKV * kVRow;
   static constexpr int kVOff = kNStage * kKTileB;
-  static constexpr int kLds = kVOff + kNStage * kVTileB;
+  static constexpr int kLds = kVOff + kNStage * kVTileB;  // of one key group
   // 1 KiB DMA instructions per wave per tile
-  static constexpr int kKLoads = kKTileB / 1024 / kNW;
-  static constexpr int kVLoads = kVTileB / 1024 / kNW;
+  static constexpr int kKLoads = kKTileB / 1024 / R;
+  static constexpr int kVLoads = kVTileB / 1024 / R;
   static constexpr int kLoadsPerTile = kKLoads + kVLoads;
   static constexpr int kSteps = D / 16;  // k-steps of a bf16 QK product
   static constexpr int kNB = D / 32;     // 32-channel output blocks
@@ -211,18 +215,26 @@ __device__ __forceinline__ float softmax_fixup(f32x16 (&s)[2], f32x16 (&sn)[2],
 
 }  // namespace
 
-template <int D, bool QK8, bool SPARSE, bool VT>
-__global__ __launch_bounds__(kNW * 64) void flash_attn_kernel(FlashParams p) {
-  // head dim 64 runs the dense bf16 row-major-V form only
-  static_assert(D == 128 || (D == 64 && !QK8 && !SPARSE && !VT),
-                "unsupported head dim / variant");
-  using L = Stage<D, QK8>;
+template <int D, bool QK8, bool SPARSE, bool VT, int R, int G>
+__global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p) {
+  // head dim 64 runs the dense bf16 row-major-V form only, row blocks of
+  // fewer wavefronts the dense bf16 one
+  static_assert(D == 128 || (!QK8 && !SPARSE && !VT), "unsupported variant");
+  static_assert(R == 8 || (!QK8 && !SPARSE), "unsupported variant");
+  static_assert(R * G == 8 || (R == 4 && G == 1), "8 wavefronts per CU");
+  using L = Stage<D, QK8, R>;
+  constexpr int BQ = R * 32;
   constexpr int NB = L::kNB;
+  constexpr int kNStage = L::kNStage;
+  constexpr int kRowsPerWave = L::kRowsPerWave;
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds_raw[];
   lds_u8* lds = (lds_u8*)lds_raw;
 
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // wave: row wavefront, grp: key group (every G-th tile of the sweep)
+  const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) % R);
+  const int grp =
+      G == 1 ? 0 : __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) / R);
   const int l32 = lane & 31;
   const int hf = lane >> 5;
 
@@ -249,7 +261,7 @@ __global__ __launch_bounds__(kNW * 64) void flash_attn_kernel(FlashParams p) {
   const uint16_t* vbase =
       VT ? p.vt + ((int64_t)b * p.Hkv + hk) * p.vt_tiles * (kBKV * D)
          : p.v + b * p.v_sb + hk * p.v_sh;
-  const int q0 = qblk * kBQ + wave * 32;
+  const int q0 = qblk * BQ + wave * 32;
   const float c = p.c;
   const int kv_end =
       resolve_len(p.kv_len_dev, p.kv_len_count, b, p.kv_end, p.Skv);
@@ -274,7 +286,7 @@ __global__ __launch_bounds__(kNW * 64) void flash_attn_kernel(FlashParams p) {
   auto tile_of = [&](int j) {
     if constexpr (SPARSE)
       return __builtin_amdgcn_readfirstlane(tiles[tbeg + j]);
-    return tbeg + j;
+    return tbeg + j * G + grp;
   };
   // outputs: a split part writes o (unnormalized), m and l of its rows to
   // the workspace, row unit*256 + (row - qblk*256)
@@ -285,12 +297,12 @@ __global__ __launch_bounds__(kNW * 64) void flash_attn_kernel(FlashParams p) {
   if (unit >= 0) {
     const int64_t units = (int64_t)p.n_tail * p.n_split;
     out32 = p.ws;
-    out_m = p.ws + units * kBQ * D;
-    out_l = out_m + units * kBQ;
+    out_m = p.ws + units * BQ * D;
+    out_l = out_m + units * BQ;
     out_o = nullptr;
   }
   auto out_row = [&](int row) -> int64_t {  // index of row in out32/m/l
-    if (unit >= 0) return (int64_t)unit * kBQ + (row - qblk * kBQ);
+    if (unit >= 0) return (int64_t)unit * BQ + (row - qblk * BQ);
     return ((int64_t)b * p.Hq + h) * p.Sq + row;
   };
   // an empty table row, or a split part past a runtime kv_len: nothing to
@@ -315,6 +327,10 @@ __global__ __launch_bounds__(kNW * 64) void flash_attn_kernel(FlashParams p) {
     }
     return;
   }
+
+  // tiles of this key group, and barriers the longest group takes
+  const int niter = (ntiles + G - 1) / G;
+  ntiles = (ntiles - grp + G - 1) / G;
 
   // ---- Q^T operands, in registers for the whole sweep: lane holds row
   // q0 + l32, channels 16t + 8hf .. +8 for step t.  They are pre-scaled by
@@ -374,7 +390,8 @@ __global__ __launch_bounds__(kNW * 64) void flash_attn_kernel(FlashParams p) {
     }
   }
 
-  // ---- tile loads: wave w fills rows 8w .. 8w+7 of the K and V tiles;
+  // ---- tile loads: wave w fills rows 8w .. 8w+7 (of 4 wavefronts: 16w ..
+  // 16w+15) of the K and V tiles;
   // lane -> (row, physical chunk).  256-byte rows (bf16 K and V at
   // D = 128): 4 rows per 1 KiB instruction, K chunk c of key r at
   // c ^ (r & 15), V chunk c at c ^ (4 * (r & 3)).  128-byte rows (E4M3 K,
@@ -395,16 +412,20 @@ __global__ __launch_bounds__(kNW * 64) void flash_attn_kernel(FlashParams p) {
         kvo[i] = row * krow + (((lane & 15) ^ (row & 15)) * 16);
       }
     } else {
-      const int row = wave * kRowsPerWave + (lane >> 3);
-      kvo[0] = row * krow + (((lane & 7) ^ ((row >> 1) & 7)) * 16);
+#pragma unroll
+      for (int i = 0; i < L::kKLoads; ++i) {
+        const int row = wave * kRowsPerWave + i * 8 + (lane >> 3);
+        kvo[i] = row * krow + (((lane & 7) ^ ((row >> 1) & 7)) * 16);
+      }
     }
     if constexpr (VT) {
       // packed V tile: 128 channel rows x 128 B (64 keys); wave w fills
-      // rows 16w .. 16w+15, 8 rows per instruction; chunk c of row d at
-      // c ^ ((d >> 1) & 7), as the E4M3 K tile
+      // rows 16w .. 16w+15 (of 4 wavefronts: 32w .. 32w+31), 8 rows per
+      // instruction; chunk c of row d at c ^ ((d >> 1) & 7), as the E4M3 K
+      // tile
 #pragma unroll
       for (int i = 0; i < L::kVLoads; ++i) {
-        const int row = wave * 16 + i * 8 + (lane >> 3);
+        const int row = wave * (128 / R) + i * 8 + (lane >> 3);
         vvo[i] = row * vrow + (((lane & 7) ^ ((row >> 1) & 7)) * 16);
       }
     } else if constexpr (L::kVRow == 256) {
@@ -414,64 +435,77 @@ __global__ __launch_bounds__(kNW * 64) void flash_attn_kernel(FlashParams p) {
         vvo[i] = row * vrow + (((lane & 15) ^ (4 * (row & 3))) * 16);
       }
     } else {
-      const int row = wave * kRowsPerWave + (lane >> 3);
-      vvo[0] = row * vrow + (((lane & 7) ^ (4 * ((row >> 1) & 1))) * 16);
+#pragma unroll
+      for (int i = 0; i < L::kVLoads; ++i) {
+        const int row = wave * kRowsPerWave + i * 8 + (lane >> 3);
+        vvo[i] = row * vrow + (((lane & 7) ^ (4 * ((row >> 1) & 1))) * 16);
+      }
     }
   }
-  const uint32_t lds_k = (uint32_t)(uintptr_t)lds +
+  const uint32_t lds_k = (uint32_t)(uintptr_t)lds + (uint32_t)grp * L::kLds +
                          (uint32_t)wave * (kRowsPerWave * L::kKRow);
-  // (a packed V tile's wave share, 16 rows of 128 B, is 8 rows of 256 B)
-  const uint32_t lds_v = (uint32_t)(uintptr_t)lds + L::kVOff +
+  // (a packed V tile's wave share of 128-byte rows is as many bytes)
+  const uint32_t lds_v = (uint32_t)(uintptr_t)lds + (uint32_t)grp * L::kLds + L::kVOff +
                          (uint32_t)wave * (kRowsPerWave * L::kVRow);
-  // t: position in the visit order (selects the LDS stage); kt: key tile
-  // The request of the tile at visit position t (key tile kt): descriptors
-  // and LDS stages.  An invalid request (past the last tile) has empty
-  // ranges: its DMAs read nothing and fill their stage with zeros.
+  // One tile's request, K or V: its descriptor and LDS stage, for visit
+  // position t (which selects the stage) and key tile kt.  An invalid
+  // request (past the last tile) has an empty range: its DMAs read nothing
+  // and fill their stage with zeros.
   struct TileReq {
-    u32x4 rk, rv;
-    uint32_t sk, sv;
+    u32x4 rsrc;
+    uint32_t lds;
   };
-  auto tile_req = [&](bool valid, int t, int kt) {
-    const int kv0 = kt * kBKV;
-    int rows = kv_end - kv0 < kBKV ? kv_end - kv0 : kBKV;
+  auto tile_rows = [&](bool valid, int kt) {
+    int rows = kv_end - kt * kBKV < kBKV ? kv_end - kt * kBKV : kBKV;
     // a listed tile may start past kv_end; readfirstlane keeps the clamp,
     // which the compiler forms as a vector med3, out of the scalar descriptor
     if constexpr (SPARSE) rows = __builtin_amdgcn_readfirstlane(rows < 0 ? 0 : rows);
-    if (!valid) rows = 0;
-    TileReq r;
-    r.rk = make_rsrc((uint64_t)(uintptr_t)kbase + (uint64_t)kv0 * krow,
-                     (uint32_t)rows * krow);
+    return valid ? (uint32_t)rows : 0u;
+  };
+  auto req_k = [&](bool valid, int t, int kt) {
+    return TileReq{make_rsrc((uint64_t)(uintptr_t)kbase +
+                                 (uint64_t)(kt * kBKV) * krow,
+                             tile_rows(valid, kt) * krow),
+                   lds_k + (uint32_t)(t % kNStage) * L::kKTileB};
+  };
+  auto req_v = [&](bool valid, int t, int kt) {
     // a packed V tile is one contiguous 16 KiB block, zero past kv_end
-    r.rv = VT ? make_rsrc((uint64_t)(uintptr_t)vbase + (uint64_t)kt * L::kVTileB,
-                          valid ? (uint32_t)L::kVTileB : 0u)
-              : make_rsrc((uint64_t)(uintptr_t)vbase + (uint64_t)kv0 * vrow,
-                          (uint32_t)rows * vrow);
-    r.sk = lds_k + (uint32_t)(t % kNStage) * L::kKTileB;
-    r.sv = lds_v + (uint32_t)(t % kNStage) * L::kVTileB;
-    return r;
+    return TileReq{
+        VT ? make_rsrc((uint64_t)(uintptr_t)vbase + (uint64_t)kt * L::kVTileB,
+                       valid ? (uint32_t)L::kVTileB : 0u)
+           : make_rsrc((uint64_t)(uintptr_t)vbase + (uint64_t)(kt * kBKV) * vrow,
+                       tile_rows(valid, kt) * vrow),
+        lds_v + (uint32_t)(t % kNStage) * L::kVTileB};
   };
-  // DMA instruction `part` of a request: the K parts first (K is read one
-  // phase earlier than V: 0.25-0.45 % at V7 against interleaving the two)
-  auto dma_part = [&](const TileReq& r, int part) {
+  auto dma_k = [&](const TileReq& r, int i) {
+    lds_dma16_buf(r.rsrc, kvo[i], r.lds + i * 1024);
+  };
+  auto dma_v = [&](const TileReq& r, int i) {
+    lds_dma16_buf(r.rsrc, vvo[i], r.lds + i * 1024);
+  };
+  // DMA instruction `part` of an iteration's requests: the K parts first (K
+  // is read one phase earlier than V: 0.25-0.45 % at V7 against interleaving
+  // the two)
+  auto dma_part = [&](const TileReq& rk, const TileReq& rv, int part) {
     if (part < L::kKLoads)
-      lds_dma16_buf(r.rk, kvo[part], r.sk + part * 1024);
+      dma_k(rk, part);
     else
-      lds_dma16_buf(r.rv, vvo[part - L::kKLoads],
-                    r.sv + (part - L::kKLoads) * 1024);
+      dma_v(rv, part - L::kKLoads);
   };
-  auto issue_tile = [&](int t, int kt) {
-    const TileReq r = tile_req(true, t, kt);
+  auto issue_k = [&](int t) {
+    const TileReq r = req_k(t < ntiles, t, t < ntiles ? tile_of(t) : 0);
 #pragma unroll
-    for (int i = 0; i < L::kLoadsPerTile; ++i) dma_part(r, i);
+    for (int i = 0; i < L::kKLoads; ++i) dma_k(r, i);
   };
-  // wait until at most `pending` tiles of this wave's loads are in flight,
-  // then make every wave's loads visible
-  auto wait_tiles = [&](int pending) {
-    wait_vmcnt(pending * L::kLoadsPerTile);
-    __syncthreads();
+  auto issue_v = [&](int t) {
+    const TileReq r = req_v(t < ntiles, t, t < ntiles ? tile_of(t) : 0);
+#pragma unroll
+    for (int i = 0; i < L::kVLoads; ++i) dma_v(r, i);
   };
 
-  // ---- per-lane LDS operand offsets (bytes within a stage)
+  // ---- per-lane LDS operand offsets (bytes within a stage, plus the key
+  // group's ring)
+  const int gbase = grp * L::kLds;
   // K: step t, key block kb: row kb*32 + l32, chunk 2t + hf (kb adds 8 KiB)
   // E4M3 K: step t (64 channels), half e: row kb*32 + l32, chunk
   // 4t + 2hf + e (kb adds 4 KiB)
@@ -480,10 +514,11 @@ __global__ __launch_bounds__(kNW * 64) void flash_attn_kernel(FlashParams p) {
   int kread[L::kSteps];
 #pragma unroll
   for (int t = 0; t < L::kSteps; ++t)
-    kread[t] = QK8 ? l32 * 128 +
-                         ((((t >> 1) * 4 + 2 * hf + (t & 1)) ^ ((l32 >> 1) & 7)) * 16)
-             : L::kKRow == 256 ? l32 * 256 + (((2 * t + hf) ^ (l32 & 15)) * 16)
-                               : l32 * 128 + (((2 * t + hf) ^ ((l32 >> 1) & 7)) * 16);
+    kread[t] = gbase +
+               (QK8 ? l32 * 128 +
+                          ((((t >> 1) * 4 + 2 * hf + (t & 1)) ^ ((l32 >> 1) & 7)) * 16)
+                : L::kKRow == 256 ? l32 * 256 + (((2 * t + hf) ^ (l32 & 15)) * 16)
+                                  : l32 * 128 + (((2 * t + hf) ^ ((l32 >> 1) & 7)) * 16));
   // V^T: channel block mb, key step u (adds 4 KiB), read half e (adds 2 KiB)
   // Packed V: key step u, channel block mb (adds 4 KiB): row 32mb + l32,
   // logical chunk 2u + hf, at physical chunk (2u + hf) ^ ((l32 >> 1) & 7)
@@ -492,7 +527,7 @@ __global__ __launch_bounds__(kNW * 64) void flash_attn_kernel(FlashParams p) {
     const int sw = (l32 >> 1) & 7;
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      vread[u] = L::kVOff + l32 * 128 + (((2 * u + hf) ^ sw) * 16);
+      vread[u] = gbase + L::kVOff + l32 * 128 + (((2 * u + hf) ^ sw) * 16);
   } else {
     const int g = lane >> 4, j16 = lane & 15;
     const int vkey = 4 * (g >> 1) + (j16 >> 2);
@@ -503,8 +538,8 @@ __global__ __launch_bounds__(kNW * 64) void flash_attn_kernel(FlashParams p) {
 #pragma unroll
     for (int mb = 0; mb < NB; ++mb) {
       const int d0 = 32 * mb + vd0;
-      vread[mb] = L::kVOff + vkey * L::kVRow + (((d0 >> 3) ^ vsw) * 16) +
-                  (d0 & 7) * 2;
+      vread[mb] = gbase + L::kVOff + vkey * L::kVRow +
+                  (((d0 >> 3) ^ vsw) * 16) + (d0 & 7) * 2;
     }
   }
 
@@ -691,11 +726,22 @@ __global__ __launch_bounds__(kNW * 64) void flash_attn_kernel(FlashParams p) {
 
 
 
-  // ---- prologue: tiles 0 .. kDist-1 requested, S(0)
+  // ---- prologue: the tiles the iterations before the first would have
+  // requested, S(0)
+  if constexpr (R == 8) {
 #pragma unroll
-  for (int t = 0; t < kDist; ++t)
-    if (t < ntiles) issue_tile(t, tile_of(t));
-  wait_tiles(ntiles - 1 < kDist - 1 ? ntiles - 1 : kDist - 1);
+    for (int t = 0; t < kDist; ++t) {
+      issue_k(t);
+      issue_v(t);
+    }
+    wait_vmcnt_c<L::kLoadsPerTile>();  // tile 0 landed
+  } else {
+    issue_k(0);
+    issue_v(0);
+    issue_k(1);
+    wait_vmcnt_c<L::kLoadsPerTile>();  // K(0) landed
+  }
+  __syncthreads();
   f32x16 sA[2], sB[2];
   phase_a(F{}, IC<0>{}, sA, sA, no_dma);
   {
@@ -716,27 +762,30 @@ __global__ __launch_bounds__(kNW * 64) void flash_attn_kernel(FlashParams p) {
     // table reads first: their wait joins the tile wait below
     const int k_next = has_next ? tile_of(jt + 1) * kBKV : 0;
     const int t_issue = jt + kDist < ntiles ? tile_of(jt + kDist) : 0;
-    {
-      int pend = ntiles - 1 - (jt + 1);
-      if (pend > kDist - 2) pend = kDist - 2;
-      if (pend < 0) pend = 0;
-      wait_tiles(pend);  // tile jt+1 resident; tile jt-1's stage is free
-    }
+    // tile jt+1 resident (of 4 wavefronts: K of tile jt+1 and V of tile jt)
+    // and every wave done with iteration jt-1: the loads of the iteration
+    // before were issued that long ago, nothing younger is in flight
+    wait_vmcnt_c<0>();
+    __syncthreads();
     // Tile jt+kDist goes into the stage tile jt-2 used (free since the
     // barrier above), its DMA instructions spread over phase A's MFMAs:
     // part p beside MFMA floor((2p+1) NM / 2P).  Issued together after the
     // barrier, the workgroup's 32 queued at the CU's address unit, and the
     // wavefronts, issuing in order, waited behind theirs with their MFMAs
     // stalled.  Past the last tile the request is empty (no branch inside
-    // the interleaved phase; the epilogue drains it).
-    const TileReq req = tile_req(jt + kDist < ntiles, jt + kDist, t_issue);
+    // the interleaved phase; the epilogue drains it).  Of 4 wavefronts, K of
+    // tile jt+2 goes into the stage of K(jt), whose scores are done, and V
+    // of tile jt+1 into the stage of V(jt-1).
+    const TileReq rk = req_k(jt + kDist < ntiles, jt + kDist, t_issue);
+    const TileReq rv =
+        R == 8 ? req_v(jt + kDist < ntiles, jt + kDist, t_issue)
+                : req_v(has_next, jt + 1, k_next / kBKV);  // (k_next: tile jt+1)
     constexpr int NM = QK8 ? 4 : 2 * L::kSteps, NP = L::kLoadsPerTile;
     auto dma = [&](int i) {
 #pragma unroll
       for (int part = 0; part < NP; ++part)
-        if (i == (2 * part + 1) * NM / (2 * NP)) dma_part(req, part);
+        if (i == (2 * part + 1) * NM / (2 * NP)) dma_part(rk, rv, part);
     };
-    auto dma_b = no_dma;
     // second half of tile jt (first half already in pw, its sum in hsum)
     // (On the last tile the QK product runs on a stale or zero-filled LDS
     // stage and its scores are never used.  Selecting softmax_half there
@@ -752,26 +801,74 @@ __global__ __launch_bounds__(kNW * 64) void flash_attn_kernel(FlashParams p) {
     // stale contents of sn into pw words that nothing reads afterwards: one
     // phase-B body in the loop keeps its register allocation within the
     // 256 VGPRs of two wavefronts per SIMD (two bodies spilled).
-    phase_b(T{}, IC<S>{}, sn, hsum, dma_b);
+    phase_b(T{}, IC<S>{}, sn, hsum, no_dma);
   };
 
-  int jt = 0;
-  static_assert(kNStage == 4, "the key loop is unrolled over the ring");
-  for (; jt < ntiles; jt += 4) {
+  // the key loop is unrolled over the ring
+  for (int jt = 0; jt < ntiles; jt += kNStage) {
     iteration(IC<0>{}, jt, sA, sB);
     if (jt + 1 >= ntiles) break;
     iteration(IC<1>{}, jt + 1, sB, sA);
-    if (jt + 2 >= ntiles) break;
-    iteration(IC<2>{}, jt + 2, sA, sB);
-    if (jt + 3 >= ntiles) break;
-    iteration(IC<3>{}, jt + 3, sB, sA);
+    if constexpr (kNStage == 4) {
+      if (jt + 2 >= ntiles) break;
+      iteration(IC<2>{}, jt + 2, sA, sB);
+      if (jt + 3 >= ntiles) break;
+      iteration(IC<3>{}, jt + 3, sB, sA);
+    }
   }
+
+  // the barriers of the iterations that only longer key groups have
+  if constexpr (G > 1)
+    for (int j = ntiles; j < niter; ++j) __syncthreads();
 
   // the empty requests of the last iterations still write their stages
   // (zeros), one of them a stage the epilogue stages o through: drain every
   // wave's before any wave writes there
   wait_vmcnt(0);
   __syncthreads();
+
+  // ---- key groups: groups 1 .. G-1 leave their o, m, l in LDS and end,
+  // group 0 takes them in, in LSE space as kernels/splash.py:653-662 merges
+  // residuals.  A group without tiles has weight 0 (group 0 always has one).
+  if constexpr (G > 1) {
+    constexpr int kPart = D * 32 * 4 + 512;  // bytes of a wavefront's o, m, l
+    static_assert((G - 1) * R * kPart <= G * L::kLds, "parts fit the rings");
+    typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
+    typedef __attribute__((address_space(3))) float lds_f32;
+    if (grp > 0) {
+      lds_u8* part_o = lds + ((grp - 1) * R + wave) * kPart;
+#pragma unroll
+      for (int mb = 0; mb < NB; ++mb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          *(lds_f32x4*)(part_o + (mb * 4 + j) * 1024 + lane * 16) =
+              f32x4{o[mb][4 * j], o[mb][4 * j + 1], o[mb][4 * j + 2], o[mb][4 * j + 3]};
+      *(lds_f32*)(part_o + D * 128 + lane * 4) = ntiles > 0 ? m : -INFINITY;
+      *(lds_f32*)(part_o + D * 128 + 256 + lane * 4) = ntiles > 0 ? l : 0.f;
+    }
+    __syncthreads();
+    if (grp > 0) return;
+#pragma unroll
+    for (int g = 1; g < G; ++g) {
+      const lds_u8* part_o = lds + ((g - 1) * R + wave) * kPart;
+      const float mg = *(const lds_f32*)(part_o + D * 128 + lane * 4);
+      const float lg = *(const lds_f32*)(part_o + D * 128 + 256 + lane * 4);
+      const float mx = fmaxf(m, mg);
+      const float w0 = __builtin_amdgcn_exp2f(m - mx);
+      const float wg = __builtin_amdgcn_exp2f(mg - mx);
+      m = mx;
+      l = l * w0 + lg * wg;
+#pragma unroll
+      for (int mb = 0; mb < NB; ++mb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const f32x4 x = *(const lds_f32x4*)(part_o + (mb * 4 + j) * 1024 + lane * 16);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            o[mb][4 * j + e] = o[mb][4 * j + e] * w0 + x[e] * wg;
+        }
+    }
+  }
 
   // ---- epilogue: lane holds row q0 + l32, channels 32mb + 8g + 4hf + e
   const float ltot = l + __shfl_xor(l, 32, 64);
@@ -789,26 +886,20 @@ __global__ __launch_bounds__(kNW * 64) void flash_attn_kernel(FlashParams p) {
   // writes 16 bytes (fp32: 32) into each of 32 rows, so a wave's rows take
   // 16 instructions touching 32 lines each.  Each wave instead writes its
   // rows, one pass of RB-byte row slices at a time, into a private 32 x RB
-  // region of a ring stage the last iteration does not read (stages
-  // (jl+2)%4 and (jl+3)%4; the drain above left no DMA pending), reads them back as
-  // whole slices and stores 16 contiguous bytes per lane.  16-byte chunk j
-  // of slice row r sits at chunk j ^ (r % (RB/16)).  bf16 K stages hold
-  // two regions of RB = 2D bytes (bf16 o in one pass, fp32 o in two); with
-  // E4M3 keys the regions are 128-byte slices in the two free V stages
-  // (bf16 o in two passes, fp32 o in four).
+  // region of the K ring, which nothing reads or fills after the drain
+  // above, reads them back as whole slices and stores 16 contiguous bytes
+  // per lane.  16-byte chunk j of slice row r sits at chunk j ^ (r % (RB/16)).
+  // bf16 K stages hold regions of RB = 2D bytes a row (bf16 o in one pass,
+  // fp32 o in two); with E4M3 keys the slices are 128 bytes (bf16 o in two
+  // passes, fp32 o in four).
   constexpr int RB = QK8 ? 128 : 2 * D;  // slice bytes per row
   constexpr int NCH = RB / 16;           // 16-byte chunks per slice
   constexpr int RPI = 64 / NCH;          // rows per read-back instruction
-  constexpr int WPS = QK8 ? 4 : 2;       // wave regions per stage
-  static_assert((QK8 ? L::kVTileB : L::kKTileB) >= WPS * 32 * RB &&
-                    L::kVTileB >= WPS * 32 * RB,
-                "a stage holds its wave regions");
-  const int jl = ntiles - 1;
-  const int grp = wave / WPS;  // QK8: V stages 0, 1; else K 0, 1, V 0, 1
-  const int st = (jl + 2 + (grp & 1)) & 3;
-  lds_u8* reg = lds + ((QK8 || grp >= 2) ? L::kVOff + st * L::kVTileB
-                                         : st * L::kKTileB) +
-                (wave % WPS) * (32 * RB);
+  // (behind the key groups' parts, which other wavefronts may still read)
+  constexpr int kReg = G > 1 ? (G - 1) * R * (D * 32 * 4 + 512) : 0;
+  static_assert(kReg + R * 32 * RB <= G * L::kLds && kReg % 16 == 0,
+                "the rings hold the wave regions");
+  lds_u8* reg = lds + kReg + wave * (32 * RB);
   // (lane laundered through an empty asm: the compiler otherwise shares
   // these swizzled offsets with the key-operand offsets, computes them
   // before the key loop and spills them across it)
@@ -958,11 +1049,12 @@ __global__ __launch_bounds__(256) void split_merge_kernel(FlashParams p) {
   }
 }
 
-template <int D, bool QK8, bool SPARSE, bool VT>
+template <int D, bool QK8, bool SPARSE, bool VT, int R, int G>
 static int launch_flash(const FlashParams& base, hipStream_t st) {
-  using L = Stage<D, QK8>;
+  using L = Stage<D, QK8, R>;
+  constexpr int BQ = R * 32;
   FlashParams p = base;
-  p.n_qblk = (p.Sq + kBQ - 1) / kBQ;
+  p.n_qblk = (p.Sq + BQ - 1) / BQ;
   const int64_t nwg = (int64_t)p.n_qblk * p.Hq * p.B;
   if (nwg > 0x7fffffff)
     return set_error(DT_ERR_SHAPE, "dt_flash_fwd: grid too large");
@@ -975,18 +1067,18 @@ static int launch_flash(const FlashParams& base, hipStream_t st) {
   if (p.n_split > kMaxSplit)  // the planner stays within it; the merge relies on it
     return set_error(DT_ERR_ARG, "dt_flash_fwd: %d split parts > %d",
                      p.n_split, kMaxSplit);
-  if (p.ws == nullptr || p.n_split <= 1) {
+  if (R != 8 || p.ws == nullptr || p.n_split <= 1) {
     p.n_split = 1;
     p.n_tail = 0;
     p.n_main = p.n_wg;
   }
-  const void* fn = (const void*)flash_attn_kernel<D, QK8, SPARSE, VT>;
+  const void* fn = (const void*)flash_attn_kernel<D, QK8, SPARSE, VT, R, G>;
   static std::atomic<uint64_t> lds_set{0};
-  if (int rc = ensure_lds_limit(fn, L::kLds, lds_set, "dt_flash_fwd"))
+  if (int rc = ensure_lds_limit(fn, G * L::kLds, lds_set, "dt_flash_fwd"))
     return rc;
   const int grid = p.n_main + p.n_tail * p.n_split;
-  hipLaunchKernelGGL((flash_attn_kernel<D, QK8, SPARSE, VT>), dim3(grid),
-                     dim3(kNW * 64), L::kLds, st, p);
+  hipLaunchKernelGGL((flash_attn_kernel<D, QK8, SPARSE, VT, R, G>), dim3(grid),
+                     dim3(R * G * 64), G * L::kLds, st, p);
   if (p.n_tail > 0) {
     const dim3 mg(p.n_tail * (kBQ / (256 / (D / 4))));
     if (p.n_split <= 2)
@@ -1010,6 +1102,10 @@ SplitPlan split_plan(int64_t n_wg, int ntiles, int n_cu, int D, size_t max_ws) {
   if (n_cu <= 0 || n_wg <= 0) return sp;
   const int64_t rem = n_wg % n_cu;
   if (rem == 0) return sp;
+  // Short sweeps over many rounds: the idle CUs of the last one are a few
+  // percent of the call at most, about what the split's second launch costs
+  // (H40 Sq 48360, 8 tiles, 29.8 rounds: 610 us with it, 606 without).
+  if (ntiles <= 16 && n_wg >= 8 * (int64_t)n_cu) return sp;
   // The last round's rem query blocks cut into ns parts run as
   // ceil(rem * ns / n_cu) rounds of parts of ntiles / ns tiles; each
   // workgroup also pays a start-up (q load, the first tiles' latency, the
@@ -1064,26 +1160,98 @@ int device_cu_count(int* n_cu) {
   return DT_OK;
 }
 
+// Workgroup shape of a dense bf16 launch: R row wavefronts
+// (32 query rows each) times G key groups.  8 x 1 is the shape for long
+// sweeps and full grids.  With few query blocks or few key tiles a
+// workgroup's start-up, the tail split's second launch and the idle CUs cost
+// more than the tile DMA that smaller row blocks repeat:
+//   4 x 1  128 rows; one wavefront per SIMD, two workgroups per CU, one
+//          computing while the other starts or ends;
+//   4 x 2  128 rows, the tiles dealt to two key groups merged in LDS;
+//   2 x 4  64 rows, four key groups (head dim 64: four rings fit the LDS).
+// The estimate below is microseconds on one MI355X, fitted to N(0,1) calls
+// captured in a graph (start-up and gap to the next launch included): `own`
+// a lone workgroup per CU, `shared` two per CU, for a sweep of T tiles.
+// Measured, D = 128, before (8 x 1 and its split) -> chosen: H8 S512
+// 17.0 -> 12.4 us, H24 S512 22.3 -> 12.9, H24 S1024 30.4 -> 21.2, H8 S2048
+// 33.6 -> 29.6, H96 S1024 70.1 -> 57.5; kept 8 x 1: H2 S4096 (split 10 ways)
+// 33.8 against 49.5, H24 S2048 52.4 against 57.6.  D = 64: H8 S1024
+// 16.3 -> 10.6, H16 S2048 29.7 -> 24.6, kept H8 S4096 44.9 against 47.0.
+struct RowShape {
+  int r, g;
+};
+
+RowShape row_shape(const FlashParams& p, int D, int n_cu) {
+  const double T = (p.kv_end + kBKV - 1) / kBKV;
+  auto blocks = [&](int rows) {
+    return (int64_t)p.B * p.Hq * ((p.Sq + rows - 1) / rows);
+  };
+  const bool d64 = D == 64;
+  // 8 x 1: whole rounds, then the last one (split or not)
+  const double whole = d64 ? 8 + 0.95 * T : 9 + 1.6 * T;
+  const int64_t n8 = blocks(256);
+  double best;
+  if (p.ws != nullptr && p.n_split > 1) {
+    const int64_t tail_rounds =
+        ((int64_t)p.n_tail * p.n_split + n_cu - 1) / n_cu;
+    best = (double)(p.n_main / n_cu) * whole +
+           (double)tail_rounds * ((d64 ? 0.95 : 1.6) * T / p.n_split) +
+           (d64 ? 16 : 20);
+  } else {
+    best = (double)((n8 + n_cu - 1) / n_cu) * (n8 <= n_cu ? 0.9 : 1.0) * whole;
+  }
+  RowShape shape{8, 1};
+  auto consider = [&](double cost, int r, int g) {
+    if (cost < best) {
+      best = cost;
+      shape = RowShape{r, g};
+    }
+  };
+  const int64_t n4 = blocks(128), per_cu = (n4 + n_cu - 1) / n_cu;
+  const double own = d64 ? 4.5 + 0.65 * T : 5.6 + 0.83 * T;
+  const double shared = d64 ? 4.5 + 1.07 * T : 5.6 + 1.75 * T;
+  consider((double)(per_cu / 2) * shared + (double)(per_cu % 2) * own, 4, 1);
+  if (!p.key_groups) return shape;
+  if (n4 <= n_cu) consider(d64 ? 6.0 + 0.46 * T : 7.5 + 0.72 * T, 4, 2);
+  if (d64 && blocks(64) <= n_cu) consider(6.5 + 0.26 * T, 2, 4);
+  return shape;
+}
+
+template <int D, bool VT>
+static int launch_dense(const FlashParams& p, int n_cu, hipStream_t st) {
+  const RowShape w = row_shape(p, D, n_cu);
+  if constexpr (D == 64)
+    if (w.r == 2) return launch_flash<D, false, false, VT, 2, 4>(p, st);
+  if (w.g == 2) return launch_flash<D, false, false, VT, 4, 2>(p, st);
+  if (w.r == 4) return launch_flash<D, false, false, VT, 4, 1>(p, st);
+  return launch_flash<D, false, false, VT, 8, 1>(p, st);
+}
+
 template <bool QK8, bool SPARSE>
 static int launch_d128_v(const FlashParams& p, hipStream_t st) {
-  return p.vt != nullptr ? launch_flash<128, QK8, SPARSE, true>(p, st)
-                         : launch_flash<128, QK8, SPARSE, false>(p, st);
+  return p.vt != nullptr ? launch_flash<128, QK8, SPARSE, true, 8, 1>(p, st)
+                         : launch_flash<128, QK8, SPARSE, false, 8, 1>(p, st);
 }
 
 int launch_flash_attn(const FlashParams& p, int D, hipStream_t st) {
+  int n_cu = 0;
+  if (int rc = device_cu_count(&n_cu)) return rc;
   if (D == 64) {
     if (p.k8 != nullptr || p.vt != nullptr || p.tile_span != nullptr)
       return set_error(DT_ERR_UNSUPPORTED,
                        "dt_flash_fwd: head dim 64 takes bf16 keys, row-major "
                        "V and no tile table");
-    return launch_flash<64, false, false, false>(p, st);
+    return launch_dense<64, false>(p, n_cu, st);
   }
   const bool sparse = p.tile_span != nullptr;
   if (p.k8 != nullptr)
     return sparse ? launch_d128_v<true, true>(p, st)
                   : launch_d128_v<true, false>(p, st);
-  return sparse ? launch_d128_v<false, true>(p, st)
-                : launch_d128_v<false, false>(p, st);
+  if (sparse) return launch_d128_v<false, true>(p, st);
+  // (packed and row-major V take the same shape: their results are equal
+  // bit for bit)
+  return p.vt != nullptr ? launch_dense<128, true>(p, n_cu, st)
+                         : launch_dense<128, false>(p, n_cu, st);
 }
 
 }  // namespace dt

@@ -45,6 +45,10 @@ struct FlashParams {
   // n_tail = 0 when there is no split.
   float* ws;
   int n_main, n_split, n_tail;
+  // the tiles of a block may be dealt to key groups of one workgroup (their
+  // merge rounds as the tail split does; the entry points without a
+  // workspace argument keep one order of tiles)
+  bool key_groups;
   int64_t q_sb, q_sh, q_ss;
   int64_t k_sb, k_sh, k_ss;
   int64_t v_sb, v_sh, v_ss;

@@ -47,7 +47,7 @@ int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
                 const int32_t* tile_ids, float* o32, float* m, float* l,
                 void* stream, const uint16_t* vt = nullptr,
                 int64_t vt_tiles = 0, void* ws = nullptr, size_t ws_bytes = 0,
-                const int32_t* kv_len_dev = nullptr) {
+                const int32_t* kv_len_dev = nullptr, bool key_groups = false) {
   const bool resid = (o32 != nullptr) || (m != nullptr) || (l != nullptr);
   const bool packed = vt != nullptr;
   if (!q || !k || !q_strides || !k_strides ||
@@ -163,6 +163,7 @@ int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
   p.n_split = 1;
   p.n_tail = 0;
   p.n_main = 0;
+  p.key_groups = key_groups;
   // (head dim 256 runs unsplit: the workspace is not used)
   if (ws != nullptr && D != 256) {
     if (!al16(ws))
@@ -366,5 +367,5 @@ extern "C" int dt_flash_fwd_ex(
   return dt::flash_entry(q, k, k_format == 1, v, o, B, Hq, Hkv, Sq, Skv, D,
                          q_strides, k_strides, v_strides, o_strides, scale,
                          kv_len, mk, tile_span, tile_ids, o32, m, l, stream, vt,
-                         vt_tiles, workspace, workspace_bytes, kv_len_dev);
+                         vt_tiles, workspace, workspace_bytes, kv_len_dev, true);
 }

@@ -10,7 +10,9 @@ rows, one workgroup per CU, whose 128 KiB LDS ring of K/V stages it fills)
 and 64 keys per stage.  What a shape decides here is the launch plan: how
 the query blocks of a partly filled last round of workgroups are split
 over their key tiles (``launch_plan``, from ``dt_flash_fwd_plan``, the
-planner ``dt_flash_fwd_ex`` itself uses).
+planner ``dt_flash_fwd_ex`` itself uses).  Dense bf16 calls with few query
+blocks or few key tiles run in smaller row blocks instead, which the plan does
+not describe.
 
 The reference's entry points keep their names, arguments and resolution
 order (pinned, else tuned, else default), so callers that resolve blocks

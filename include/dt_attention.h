@@ -432,7 +432,9 @@ size_t dt_flash_fwd_workspace_bytes(int B, int Hq, int Sq, int Skv,
  * and never splits.  This is the gfx950 side of the reference's per-shape block
  * resolution (kernels/block_sizes.py:537-577, used at
  * kernels/mesh_attention.py:198-215): the tile is fixed, and what a shape
- * decides is the tail split.
+ * decides is the tail split.  A dense bf16 call with few query blocks or few
+ * key tiles may run in workgroups of 128 or 64 rows instead and leave the
+ * workspace unused.
  */
 int dt_flash_fwd_plan(int B, int Hq, int Sq, int Skv, int kv_len, int D,
                       size_t workspace_bytes, int32_t* plan,

@@ -1,0 +1,66 @@
+"""Workgroup shapes of the dense bf16 kernel: few query blocks or few key tiles
+run in 128- or 64-row workgroups, with the tiles dealt to key groups of one
+workgroup.  Sizes at the edges of the row blocks (64, 128, 256 rows), of the
+tiles (64 keys) and of the groups (fewer tiles than groups), against the
+float64 oracle."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_helpers import assert_attn_close, banner, seeded, to64
+from oracle import attention as A
+
+pytestmark = pytest.mark.gpu
+
+# (B, Hq, Hkv, Sq, Skv, lengths per sample or None, D)
+CASES = [(b, hq, hkv, sq, skv, n, d)
+         for d in (64, 128)
+         for b, hq, hkv, sq, skv, n in [
+             (1, 1, 1, 1, 1, None),            # one row, one key
+             (1, 2, 2, 65, 64, None),          # one tile: groups without any
+             (2, 2, 1, 129, 300, (65, 0)),     # device lengths, one of them 0
+             (1, 3, 3, 128, 1087, None),       # 17 tiles, the last of 63 keys
+             (2, 4, 2, 255, 1300, (1281, 1)),  # 21 tiles against 1
+             (1, 4, 4, 700, 2049, None),       # a last tile of one key
+         ]]
+
+
+@pytest.fixture(scope="module")
+def dta():
+  if not torch.cuda.is_available():
+    pytest.skip("no GPU")
+  import diffusers_tpu_amd
+  return diffusers_tpu_amd
+
+
+@pytest.mark.parametrize("case", CASES, ids=[str(c) for c in CASES])
+def test_row_shapes_match_oracle(dta, case):
+  b, hq, hkv, sq, skv, lens, d = case
+  banner(f"row shapes {case}")
+  q = seeded((b, hq, sq, d), 600)
+  k = seeded((b, hkv, skv, d), 601)
+  v = seeded((b, hkv, skv, d), 602)
+  n = None if lens is None else torch.tensor(lens, device="cuda",
+                                             dtype=torch.int32)
+  out = dta.attention(q, k, v, kv_len=n)
+  o, m, l = dta.residual_attention(q, k, v, kv_len=n)
+  torch.cuda.synchronize()
+  for i in range(b):
+    length = skv if lens is None else lens[i]
+    if length == 0:
+      assert not out[i].any() and not o[i].any() and not l[i].any()
+      continue
+    q64, k64, v64 = (to64(t[i:i + 1]) for t in (q, k, v))
+    want = A.attention_f64(q64, k64, v64, kv_len=length)
+    assert_attn_close(to64(out[i:i + 1]), want, f"sample {i}")
+    assert_attn_close(to64(o[i:i + 1]) / to64(l[i:i + 1]), want,
+                      f"residual {i}")
+    wo, wm, wl = A.residual_f64(q64, k64, v64, kv_len=length)
+    # m + log2(l) does not depend on the reference m: the probabilities are
+    # rounded to bf16 (2^-9 relative in l) and so is c*q (2^-9 of a score)
+    lse = to64(m[i:i + 1]) + np.log2(to64(l[i:i + 1]))
+    c = np.log2(np.e) / np.sqrt(float(d))
+    kr = np.repeat(k64[:, :, :length], hq // hkv, axis=1)
+    shift = 2.0**-9 * np.einsum("bhid,bhjd->bhij", np.abs(c * q64),
+                                np.abs(kr)).max(-1)[..., None]
+    assert (np.abs(lse - (wm + np.log2(wl))) <= shift + 2.0**-8).all()
