@@ -22,7 +22,7 @@ CALIB_PATH = PKG_DIR / "libdt_calib.so"
 SOURCES = ["capi.cpp", "qk_norm_rope.hip", "flash_fwd.hip", "flash_attn.hip",
            "flash_wide.hip",
            "row_norm.hip", "fp8_cast.hip", "v_pack.hip",
-           "k_smooth.hip"]
+           "k_smooth.hip", "merge.hip"]
 ARCH = "gfx950"
 HIPCC_FLAGS = [
     "-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",

@@ -21,6 +21,9 @@ DT_ERR_LAUNCH = -4
 
 ROPE_NONE, ROPE_HALF, ROPE_PAIR = 0, 1, 2
 
+# most parts of one dt_merge_residuals call (DT_MERGE_MAX_PARTS)
+MERGE_MAX_PARTS = 16
+
 # static scratch of dt_flash_fwd_ex_noalloc (DT_NOALLOC_SCRATCH_BYTES)
 NOALLOC_SCRATCH_BYTES = 64 << 20
 
@@ -67,6 +70,7 @@ SIGNATURES = {
     "dt_fixed_m_prepare": (_I, [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _P,
                                 _P, _I, _P, _F, _F, _I, _P, _P, _Z, _P]),
     "dt_fixed_m_prepare_workspace_bytes": (_Z, [_I] * 8),
+    "dt_merge_residuals": (_I, [_P, _P, _P, _I, _L, _I, _P, _P]),
 }
 
 _lock = threading.Lock()

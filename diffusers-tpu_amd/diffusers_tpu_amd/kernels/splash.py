@@ -41,6 +41,7 @@ Differences a caller can observe, all within the reference's tolerance:
 """
 from __future__ import annotations
 
+import ctypes
 import functools
 import math
 
@@ -476,13 +477,55 @@ def residual_attention(query, key, value, *, scale=None, block_q=None,
                  workspace=workspace)
 
 
+def _merge_kernel_ok(parts):
+  """Whether ``merge_residuals`` may call ``dt_merge_residuals`` on these
+  triples: plain contiguous float32 GPU tensors, and nothing that records,
+  transforms or traces torch operations (autograd, ``torch.func``, dispatch
+  and function modes, ``torch.compile``)."""
+  if not 1 <= len(parts) <= _lib.MERGE_MAX_PARTS or any(
+      len(p) != 3 for p in parts):
+    return False
+  ts = [t for p in parts for t in p]
+  if not all(type(t) is torch.Tensor for t in ts):
+    return False
+  if (torch.compiler.is_compiling() or
+      torch.overrides._get_current_function_mode_stack() or
+      torch.utils._python_dispatch._get_current_dispatch_mode() is not None or
+      torch._C._functorch.peek_interpreter_stack() is not None or
+      torch.autograd.forward_ad._current_level >= 0 or
+      (torch.is_grad_enabled() and any(t.requires_grad for t in ts))):
+    return False
+  o = parts[0][0]
+  shape, rows = o.shape, (*o.shape[:-1], 1)
+  return (o.dim() > 0 and o.numel() > 0 and shape[-1] % 4 == 0 and
+          all(t.is_cuda and t.device == o.device and
+              t.dtype == torch.float32 and t.is_contiguous() and
+              t.shape == (rows if i % 3 else shape) and
+              t.data_ptr() % 16 == 0 for i, t in enumerate(ts)))
+
+
 def merge_residuals(parts):
   """LSE-space merge of residual ``(o, m, l)`` triples from KV shards.
 
   The merge an outer ring loop performs (kernels/splash.py:653-664): m is a
   common scale, so ``o = sum 2^(m_i - M) o_i``, ``l = sum 2^(m_i - M) l_i``
-  with ``M = max m_i``; the normalized output is ``o / l``.
+  with ``M = max m_i``; the normalized output is ``o / l``.  What
+  ``residual_attention`` returns goes through one kernel
+  (``dt_merge_residuals``); other tensors, and calls under autograd or
+  another transform, through torch operations.
   """
+  parts = list(parts)
+  if _merge_kernel_ok(parts):
+    o = parts[0][0]
+    out = torch.empty_like(o)
+    ptrs = [(ctypes.c_void_p * len(parts))(*(p[i].data_ptr() for p in parts))
+            for i in range(3)]
+    with torch.cuda.device(o.device):
+      rc = _lib.load().dt_merge_residuals(
+          *ptrs, len(parts), o.numel() // o.shape[-1], o.shape[-1],
+          out.data_ptr(), torch.cuda.current_stream(o.device).cuda_stream)
+    _lib.check("dt_merge_residuals", rc)
+    return out
   ms = torch.stack([p[1] for p in parts])
   big = ms.max(dim=0).values
   o = sum(torch.exp2(p[1] - big) * p[0] for p in parts)

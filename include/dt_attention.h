@@ -37,6 +37,8 @@
  *   dt_flash_fwd_ex  — dt_flash_fwd / _qk8 / _blocksparse in one, V
  *                      row-major or packed, optional tail-split workspace.
  *   dt_flash_fwd_workspace_bytes — the workspace dt_flash_fwd_ex can use.
+ *   dt_merge_residuals — the LSE-space merge of residual outputs from key
+ *                      shards (kernels/splash.py:653-664).
  *   dt_flash_fwd_plan — the launch plan (grid, tail split) of a shape.
  *   dt_flash_fwd_ex_noalloc — dt_flash_fwd_ex with its workspace in static
  *                      device memory (no reference counterpart: for
@@ -528,6 +530,19 @@ int dt_fixed_m_prepare(const uint16_t* q, const uint16_t* k, uint16_t* ks,
 size_t dt_fixed_m_prepare_workspace_bytes(int B, int Hq, int Hkv, int Sq,
                                           int Skv, int D, int kv_len,
                                           int smooth);
+
+/*
+ * The LSE-space merge of `parts` residual (o, m, l) triples from key shards
+ * (kernels/splash.py:653-664): with M = max m_i,
+ *   out = sum 2^(m_i - M) o_i / sum 2^(m_i - M) l_i.
+ * o, m, l: host arrays of `parts` (1 .. DT_MERGE_MAX_PARTS) device pointers;
+ * o_i and out are contiguous fp32 [rows][D], 16-byte aligned, m_i and l_i
+ * contiguous fp32 [rows].  D a multiple of 4.
+ */
+#define DT_MERGE_MAX_PARTS 16
+int dt_merge_residuals(const float* const* o, const float* const* m,
+                       const float* const* l, int parts, int64_t rows, int D,
+                       float* out, void* stream);
 
 #ifdef __cplusplus
 }
