@@ -30,7 +30,7 @@ void clear_error() { g_msg[0] = 0; }
 //   argument is its entry count, 0/1 or B); a device length <= 0 now means
 //   no keys / rows (the empty result) instead of all of them.  Callers
 //   gate on dt_version() >= 300.
-// 0.3.1: dt_merge_residuals.
+// 0.3.1: dt_merge_residuals, dt_flash_fwd_anydim.
 extern "C" int dt_version(void) { return 301; }
 
 extern "C" const char* dt_last_error(void) { return dt::g_msg; }

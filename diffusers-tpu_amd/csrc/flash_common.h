@@ -54,6 +54,7 @@ struct FlashParams {
   int64_t v_sb, v_sh, v_ss;
   int64_t o_sb, o_sh, o_ss;
   int B, Hq, Hkv, Sq, Skv;
+  int dim;         // head dim: channels of a q, k, v, o row in memory
   int kv_end;      // keys [0, kv_end) take part (upper bound if kv_len_dev)
   // runtime key length in device memory, or null: the kernels then run with
   // resolve_len(kv_len_dev, kv_len_count, b, kv_end, Skv) keys instead of
@@ -185,6 +186,9 @@ inline int ensure_lds_limit(const void* fn, int bytes,
 
 // Launcher (flash_attn.hip): head dim D = 64 or 128.
 int launch_flash_attn(const FlashParams& p, int D, hipStream_t st);
+// Launcher (flash_dims.hip): head dims p.dim below 128, multiples of 8 other
+// than 64; bf16 keys, row-major V, no tile table.
+int launch_flash_ragged(const FlashParams& p, hipStream_t st);
 // Launcher (flash_wide.hip): head dim 256, bf16 keys, row-major V, no tile
 // table, no tail split.
 int launch_flash_wide(const FlashParams& p, hipStream_t st);
@@ -201,5 +205,12 @@ struct SplitPlan {
 SplitPlan split_plan(int64_t n_wg, int ntiles, int n_cu, int D,
                      size_t max_ws = ~size_t(0));
 int device_cu_count(int* n_cu);
+
+// Workgroup shape of a dense bf16 launch (flash_attn.hip): r row wavefronts
+// times g key groups.
+struct RowShape {
+  int r, g;
+};
+RowShape row_shape(const FlashParams& p, int D, int n_cu);
 
 }  // namespace dt

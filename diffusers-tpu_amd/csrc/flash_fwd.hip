@@ -36,8 +36,12 @@ int plan_launch(int B, int Hq, int Sq, int kv_end, int D, size_t ws_bytes,
   return DT_OK;
 }
 
-// Validation and dispatch shared by dt_flash_fwd (bf16 keys) and
-// dt_flash_fwd_qk8 (E4M3 keys, k_e4m3).
+// Channels of the kernel that runs head dim D (a multiple of 8 up to 256).
+int kernel_dim(int D) { return D <= 64 ? 64 : D <= 128 ? 128 : 256; }
+
+// Validation and dispatch shared by dt_flash_fwd (bf16 keys),
+// dt_flash_fwd_qk8 (E4M3 keys, k_e4m3) and dt_flash_fwd_anydim (any_dim: head
+// dims no kernel is built for).
 int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
                 const uint16_t* v, uint16_t* o, int B, int Hq, int Hkv, int Sq,
                 int Skv, int D, const int64_t* q_strides,
@@ -47,7 +51,8 @@ int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
                 const int32_t* tile_ids, float* o32, float* m, float* l,
                 void* stream, const uint16_t* vt = nullptr,
                 int64_t vt_tiles = 0, void* ws = nullptr, size_t ws_bytes = 0,
-                const int32_t* kv_len_dev = nullptr, bool key_groups = false) {
+                const int32_t* kv_len_dev = nullptr, bool key_groups = false,
+                bool any_dim = false) {
   const bool resid = (o32 != nullptr) || (m != nullptr) || (l != nullptr);
   const bool packed = vt != nullptr;
   if (!q || !k || !q_strides || !k_strides ||
@@ -65,9 +70,14 @@ int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
   if (Hq % Hkv)
     return set_error(DT_ERR_SHAPE, "dt_flash_fwd: Hq %d not a multiple of Hkv %d",
                      Hq, Hkv);
-  if (D != 64 && D != 128 && D != 256)
+  if (any_dim ? (D <= 0 || D % 8 || (D > 128 && D != 256))
+              : (D != 64 && D != 128 && D != 256))
     return set_error(DT_ERR_UNSUPPORTED,
-                     "dt_flash_fwd: head dim %d (supported: 64, 128, 256)", D);
+                     any_dim ? "dt_flash_fwd_anydim: head dim %d (supported: "
+                               "multiples of 8 up to 128, and 256)"
+                             : "dt_flash_fwd: head dim %d (supported: 64, 128, "
+                               "256)",
+                     D);
   if (D == 256 && (k_e4m3 || packed || tile_span != nullptr))
     return set_error(DT_ERR_UNSUPPORTED,
                      "dt_flash_fwd: head dim 256 takes bf16 keys, row-major V "
@@ -155,6 +165,7 @@ int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
   p.Hkv = Hkv;
   p.Sq = Sq;
   p.Skv = Skv;
+  p.dim = D;
   p.kv_end = (kv_len <= 0) ? Skv : kv_len;
   const float sc = (scale > 0.f) ? scale : 1.0f / sqrtf((float)D);
   p.c = sc * kLog2e;
@@ -170,7 +181,8 @@ int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
       return set_error(DT_ERR_UNSUPPORTED, "dt_flash_fwd_ex: misaligned workspace");
     int n_cu = 0;
     SplitPlan sp;
-    if (int rc = plan_launch(B, Hq, Sq, p.kv_end, D, ws_bytes, &n_cu, &sp))
+    if (int rc = plan_launch(B, Hq, Sq, p.kv_end, kernel_dim(D), ws_bytes,
+                             &n_cu, &sp))
       return rc;
     if (sp.n_split > 1 && sp.ws_bytes <= ws_bytes) {
       p.ws = (float*)ws;
@@ -180,6 +192,7 @@ int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
     }
   }
   if (D == 256) return launch_flash_wide(p, st);
+  if (D != 64 && D != 128) return launch_flash_ragged(p, st);
   return launch_flash_attn(p, D, st);
 }
 
@@ -229,6 +242,27 @@ extern "C" int dt_flash_fwd_blocksparse(
   return dt::flash_entry(q, k, k_format == 1, v, o, B, Hq, Hkv, Sq, Skv, D,
                          q_strides, k_strides, v_strides, o_strides, scale,
                          kv_len, mk, tile_span, tile_ids, o32, m, l, stream);
+}
+
+extern "C" int dt_flash_fwd_anydim(
+    const uint16_t* q, const uint16_t* k, const uint16_t* v, uint16_t* o, int B,
+    int Hq, int Hkv, int Sq, int Skv, int D, const int64_t* q_strides,
+    const int64_t* k_strides, const int64_t* v_strides,
+    const int64_t* o_strides, float scale, int kv_len,
+    const int32_t* kv_len_dev, const float* mk, float* o32, float* m, float* l,
+    void* workspace, size_t workspace_bytes, void* stream) {
+  return dt::flash_entry(q, k, false, v, o, B, Hq, Hkv, Sq, Skv, D, q_strides,
+                         k_strides, v_strides, o_strides, scale, kv_len, mk,
+                         nullptr, nullptr, o32, m, l, stream, nullptr, 0,
+                         workspace, workspace_bytes, kv_len_dev, true, true);
+}
+
+extern "C" size_t dt_flash_fwd_anydim_workspace_bytes(int B, int Hq, int Sq,
+                                                      int Skv, int kv_len,
+                                                      int D) {
+  if (D <= 0 || D % 8 || D > 256) return 0;
+  return dt_flash_fwd_workspace_bytes(B, Hq, Sq, Skv, kv_len,
+                                      dt::kernel_dim(D));
 }
 
 extern "C" size_t dt_flash_fwd_workspace_bytes(int B, int Hq, int Sq, int Skv,

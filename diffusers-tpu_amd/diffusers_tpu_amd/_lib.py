@@ -70,6 +70,10 @@ SIGNATURES = {
     "dt_fixed_m_prepare": (_I, [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _P,
                                 _P, _I, _P, _F, _F, _I, _P, _P, _Z, _P]),
     "dt_fixed_m_prepare_workspace_bytes": (_Z, [_I] * 8),
+    "dt_flash_fwd_anydim": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P,
+                                 _P, _P, _P, _F, _I, _P, _P, _P, _P, _P, _P,
+                                 _Z, _P]),
+    "dt_flash_fwd_anydim_workspace_bytes": (_Z, [_I, _I, _I, _I, _I, _I]),
     "dt_merge_residuals": (_I, [_P, _P, _P, _I, _L, _I, _P, _P]),
 }
 

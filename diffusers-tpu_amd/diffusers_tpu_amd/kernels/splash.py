@@ -26,10 +26,11 @@ Differences a caller can observe, all within the reference's tolerance:
 * As in the reference (kernels/splash.py:607-609,633), ``q * scale *
   log2(e)`` is rounded to bf16 before the QK product (the kernel does this in
   registers with one rounding).
-* Head dims: the kernels are built for 64, 128 and 256; any other multiple
-  of 8 up to 256 runs zero-padded to the next of them (zero channels change
-  no score; the extra output channels are dropped), with the scale of the
-  real dim.  Above 256 (above 128 with ``qk_fp8``) raises
+* Head dims: the kernels are built for 64, 128 and 256.  Any other multiple
+  of 8 below 128 runs as it is (``dt_flash_fwd_anydim``); those from 136 to
+  248, and with ``qk_fp8`` every dim but 128, run zero-padded to the next of
+  them (zero channels change no score; the extra output channels are
+  dropped), with the scale of the real dim.  Above 256 (above 128 with ``qk_fp8``) raises
   ``NotImplementedError``, as does a dim that is not a multiple of 8
   (kernels/splash.py:156-160).
 * ``qk_fp8`` casts K to E4M3 in one GPU pass (``fp8_cast``) and the kernel
@@ -174,7 +175,7 @@ class AttentionWorkspace:
     if packed:
       self.packed_v(packed_v_numel(b, hkv, n))
     with torch.cuda.device(self.device):
-      nbytes = _lib.load().dt_flash_fwd_workspace_bytes(
+      nbytes = _lib.load().dt_flash_fwd_anydim_workspace_bytes(
           b, hq, sq, skv, 0 if n == skv else n, d)
     if nbytes:
       self.split(nbytes)
@@ -237,6 +238,10 @@ def _launch(query, key, value, scale, kv_len, out=None, residual=False,
     if packed_v is not None:
       raise ValueError(f"packed_v is a head-dim-128 layout; head_dim={d} runs "
                        "zero-padded and packs its own V")
+    if d < 128 and not qk_fp8:
+      return _call_anydim(query, key, value, scale,
+                          n if n_dev is None else n_dev, out, residual, mk,
+                          workspace)
     # zero-padded channels: same scores, extra output channels dropped below
     res = _launch(pad_head_dim(query, kd), pad_head_dim(key, kd),
                   pad_head_dim(value, kd), scale,
@@ -269,6 +274,61 @@ def _launch(query, key, value, scale, kv_len, out=None, residual=False,
       packed_v = pack_v(v, length, out=buf)
   return _call_ex(q, k, 1 if qk_fp8 else 0, v, packed_v, out, residual,
                   hkv, skv, scale, length, mk_ptr, workspace=workspace)
+
+
+def _plain_rows(t):
+  """``_as_bf16_rows`` with rows that do not overlap (an expanded or
+  sliding-window view is copied) in a (b, h) slice below 4 GiB - 256."""
+  t = _as_bf16_rows(t)
+  s, d = t.shape[2:]
+  if (s > 1 and t.stride(2) < d) or s * t.stride(2) * 2 >= (1 << 32) - 256:
+    t = t.contiguous()
+  return t
+
+
+def _call_anydim(query, key, value, scale, n, out, residual, mk, workspace):
+  """One ``dt_flash_fwd_anydim`` call (arguments checked by ``_launch``;
+  ``n`` as in ``_call_ex``)."""
+  q, k, v = _plain_rows(query), _plain_rows(key), _plain_rows(value)
+  b, hq, sq, d = q.shape
+  _, hkv, skv, _ = k.shape
+  dev = q.device
+  if mk is not None:
+    mk = _mk_operand(mk, hq, dev)
+  n_dev = n if isinstance(n, torch.Tensor) else None
+  n_host = _lib.dev_count(n_dev) if n_dev is not None else int(n)
+  s3 = lambda t: _lib.strides3(t.stride())
+  lib = _lib.load()
+  with torch.cuda.device(dev):
+    if residual:
+      o = torch.empty((b, hq, sq, d), device=dev, dtype=torch.float32)
+      m = torch.empty((b, hq, sq, 1), device=dev, dtype=torch.float32)
+      l = torch.empty((b, hq, sq, 1), device=dev, dtype=torch.float32)
+      outs = (None, None, o.data_ptr(), m.data_ptr(), l.data_ptr())
+    else:
+      # an output that shares memory with an input is written after the call
+      direct = out is not None and all(
+          out.untyped_storage().data_ptr() != t.untyped_storage().data_ptr()
+          for t in (q, k, v))
+      o = out if direct else torch.empty((b, hq, sq, d), device=dev,
+                                         dtype=torch.bfloat16)
+      outs = (o.data_ptr(), s3(o), None, None, None)
+    nbytes = _split_bytes(b, hq, sq, skv, 0 if n_dev is not None else n_host,
+                          64 if d < 64 else 128, dev.index)
+    if not nbytes:
+      ws = None
+    elif workspace is not None:
+      ws = workspace.split(nbytes)
+    else:
+      ws = torch.empty((nbytes + 3) // 4, device=dev, dtype=torch.float32)
+    _lib.check("dt_flash_fwd_anydim", lib.dt_flash_fwd_anydim(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), outs[0], b, hq, hkv, sq, skv,
+        d, s3(q), s3(k), s3(v), outs[1], scale, n_host, _lib.ptr(n_dev),
+        _lib.ptr(mk), *outs[2:], _lib.ptr(ws), nbytes,
+        torch.cuda.current_stream(dev).cuda_stream))
+  if residual:
+    return o, m, l
+  return o if out is None else out if direct else out.copy_(o)
 
 
 @functools.lru_cache(maxsize=4096)

@@ -37,6 +37,8 @@
  *   dt_flash_fwd_ex  — dt_flash_fwd / _qk8 / _blocksparse in one, V
  *                      row-major or packed, optional tail-split workspace.
  *   dt_flash_fwd_workspace_bytes — the workspace dt_flash_fwd_ex can use.
+ *   dt_flash_fwd_anydim — dt_flash_fwd_ex at head dims that are no kernel
+ *                      width, without padded copies.
  *   dt_merge_residuals — the LSE-space merge of residual outputs from key
  *                      shards (kernels/splash.py:653-664).
  *   dt_flash_fwd_plan — the launch plan (grid, tail split) of a shape.
@@ -421,6 +423,26 @@ int dt_flash_fwd_ex(const uint16_t* q, const void* k, int k_format,
  */
 size_t dt_flash_fwd_workspace_bytes(int B, int Hq, int Sq, int Skv,
                                     int kv_len, int D);
+
+/*
+ * dt_flash_fwd_ex with bf16 keys, row-major V and no tile table, at any head
+ * dim that is a multiple of 8 up to 128 (kernels/splash.py:156-160), and 256:
+ * rows of D elements are read and written as they are, at the arithmetic of
+ * the dim itself.  Rows of one (b, h) slice of q, k, v must not overlap
+ * (stride s >= D, or one row), and a K or V slice must span less than 4 GiB -
+ * 256.  The default scale is 1/sqrt(D).
+ */
+int dt_flash_fwd_anydim(const uint16_t* q, const uint16_t* k,
+                        const uint16_t* v, uint16_t* o, int B, int Hq, int Hkv,
+                        int Sq, int Skv, int D, const int64_t* q_strides,
+                        const int64_t* k_strides, const int64_t* v_strides,
+                        const int64_t* o_strides, float scale, int kv_len,
+                        const int32_t* kv_len_dev, const float* mk, float* o32,
+                        float* m, float* l, void* workspace,
+                        size_t workspace_bytes, void* stream);
+/* Workspace bytes dt_flash_fwd_anydim can use (as the function above). */
+size_t dt_flash_fwd_anydim_workspace_bytes(int B, int Hq, int Sq, int Skv,
+                                           int kv_len, int D);
 
 /*
  * The launch plan dt_flash_fwd_ex follows for this shape on the current
