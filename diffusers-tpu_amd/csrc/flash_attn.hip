@@ -5,7 +5,8 @@
 
 namespace dt {
 
-SplitPlan split_plan(int64_t n_wg, int ntiles, int n_cu, int D, size_t max_ws) {
+SplitPlan split_plan(int64_t n_wg, int ntiles, int n_cu, int D, int bq,
+                     size_t max_ws) {
   SplitPlan sp{1, 0, (int)n_wg, 0};
   if (n_cu <= 0 || n_wg <= 0) return sp;
   const int64_t rem = n_wg % n_cu;
@@ -25,7 +26,7 @@ SplitPlan split_plan(int64_t n_wg, int ntiles, int n_cu, int D, size_t max_ws) {
   constexpr int64_t kMergeTiles = 1;  // fitted: P (16 tiles) 17.4 us at 4 parts, 19.8 at 8
   constexpr size_t kMaxWs = size_t(512) << 20;
   if (max_ws > kMaxWs) max_ws = kMaxWs;
-  const size_t unit_bytes = (size_t)kBQ * (D + 2) * sizeof(float);
+  const size_t unit_bytes = (size_t)bq * (D + 2) * sizeof(float);
   int64_t best_ns = 1, best_cost = ntiles + kStartTiles;
   for (int64_t ns = 2; ns <= kMaxSplit && ns <= ntiles / 2; ++ns) {
     if ((size_t)(rem * ns) * unit_bytes > max_ws) break;

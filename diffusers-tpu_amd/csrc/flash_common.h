@@ -36,12 +36,12 @@ struct FlashParams {
   // accumulator's order), zero past kv_end
   const uint16_t* vt;
   int64_t vt_tiles;
-  // Tail split (D = 64 and 128): workgroups [0, n_main) each run one query
+  // Tail split: workgroups [0, n_main) each run one query
   // block over all its keys; the n_tail query blocks after them run as
   // n_split parts each, one per workgroup, every part a contiguous share of
-  // the block's key tiles, writing unnormalized o, m, l for its 256 rows to
-  // ws (o: [units][256][128], then m and l: [units][256] each, units =
-  // n_tail * n_split); a merge kernel combines the parts.  n_split = 1 and
+  // the block's key tiles, writing unnormalized o, m, l for its BQ rows to ws
+  // (o: [units][BQ][D] with D the kernel's width, then m and l: [units][BQ]
+  // each, units = n_tail * n_split); a merge kernel combines the parts.  n_split = 1 and
   // n_tail = 0 when there is no split.
   float* ws;
   int n_main, n_split, n_tail;
@@ -189,11 +189,12 @@ int launch_flash_attn(const FlashParams& p, int D, hipStream_t st);
 // Launcher (flash_dims.hip): head dims p.dim below 128, multiples of 8 other
 // than 64; bf16 keys, row-major V, no tile table.
 int launch_flash_ragged(const FlashParams& p, hipStream_t st);
-// Launcher (flash_wide.hip): head dim 256, bf16 keys, row-major V, no tile
-// table, no tail split.
+// Launcher (flash_wide.hip): head dims p.dim 136 to 256, bf16 keys, row-major
+// V, no tile table.
 int launch_flash_wide(const FlashParams& p, hipStream_t st);
 
-// Tail split plan for a launch of n_wg workgroups over ntiles key
+constexpr int kMaxSplit = 16;  // most parts a query block is split into
+// Tail split plan for a launch of n_wg workgroups of bq rows over ntiles key
 // tiles on a device of n_cu compute units (one workgroup per CU): the
 // number of parts the last, partly filled round's query blocks are cut
 // into (1: no split), and the workspace bytes it needs, at most max_ws
@@ -202,7 +203,7 @@ struct SplitPlan {
   int n_split, n_tail, n_main;
   size_t ws_bytes;
 };
-SplitPlan split_plan(int64_t n_wg, int ntiles, int n_cu, int D,
+SplitPlan split_plan(int64_t n_wg, int ntiles, int n_cu, int D, int bq,
                      size_t max_ws = ~size_t(0));
 int device_cu_count(int* n_cu);
 

@@ -24,15 +24,17 @@ static bool al16(const void* ptr) { return ((uintptr_t)ptr & 15u) == 0; }
 namespace dt {
 namespace {
 
-// The tail-split plan of a launch of B * Hq * ceil(Sq / 256) query blocks
-// over kv_end keys on the current device, within ws_bytes of workspace;
+// The tail-split plan of a launch of B * Hq * ceil(Sq / 256) query blocks (128
+// rows at D = 256) over kv_end keys on the current device, within ws_bytes of
+// workspace;
 // dt_flash_fwd_ex, dt_flash_fwd_workspace_bytes and dt_flash_fwd_plan all
 // plan through here.
 int plan_launch(int B, int Hq, int Sq, int kv_end, int D, size_t ws_bytes,
                 int* n_cu, SplitPlan* sp) {
   if (int rc = device_cu_count(n_cu)) return rc;
-  const int64_t n_wg = (int64_t)B * Hq * ((Sq + 255) / 256);
-  *sp = split_plan(n_wg, (kv_end + 63) / 64, *n_cu, D, ws_bytes);
+  const int bq = D == 256 ? 128 : 256, bkv = D == 256 ? 32 : 64;
+  const int64_t n_wg = (int64_t)B * Hq * ((Sq + bq - 1) / bq);
+  *sp = split_plan(n_wg, (kv_end + bkv - 1) / bkv, *n_cu, D, bq, ws_bytes);
   return DT_OK;
 }
 
@@ -70,11 +72,11 @@ int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
   if (Hq % Hkv)
     return set_error(DT_ERR_SHAPE, "dt_flash_fwd: Hq %d not a multiple of Hkv %d",
                      Hq, Hkv);
-  if (any_dim ? (D <= 0 || D % 8 || (D > 128 && D != 256))
+  if (any_dim ? (D <= 0 || D % 8 || D > 256)
               : (D != 64 && D != 128 && D != 256))
     return set_error(DT_ERR_UNSUPPORTED,
                      any_dim ? "dt_flash_fwd_anydim: head dim %d (supported: "
-                               "multiples of 8 up to 128, and 256)"
+                               "multiples of 8 up to 256)"
                              : "dt_flash_fwd: head dim %d (supported: 64, 128, "
                                "256)",
                      D);
@@ -175,8 +177,8 @@ int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
   p.n_tail = 0;
   p.n_main = 0;
   p.key_groups = key_groups;
-  // (head dim 256 runs unsplit: the workspace is not used)
-  if (ws != nullptr && D != 256) {
+  // (dt_flash_fwd_ex runs head dim 256 unsplit: the workspace is not used)
+  if (ws != nullptr && (D != 256 || any_dim)) {
     if (!al16(ws))
       return set_error(DT_ERR_UNSUPPORTED, "dt_flash_fwd_ex: misaligned workspace");
     int n_cu = 0;
@@ -191,7 +193,7 @@ int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
       p.n_main = sp.n_main;
     }
   }
-  if (D == 256) return launch_flash_wide(p, st);
+  if (D > 128) return launch_flash_wide(p, st);
   if (D != 64 && D != 128) return launch_flash_ragged(p, st);
   return launch_flash_attn(p, D, st);
 }
@@ -260,9 +262,15 @@ extern "C" int dt_flash_fwd_anydim(
 extern "C" size_t dt_flash_fwd_anydim_workspace_bytes(int B, int Hq, int Sq,
                                                       int Skv, int kv_len,
                                                       int D) {
-  if (D <= 0 || D % 8 || D > 256) return 0;
-  return dt_flash_fwd_workspace_bytes(B, Hq, Sq, Skv, kv_len,
-                                      dt::kernel_dim(D));
+  if (D <= 0 || D % 8 || D > 256 || B <= 0 || Hq <= 0 || Sq <= 0 || Skv <= 0)
+    return 0;
+  const int kv_end = (kv_len <= 0 || kv_len > Skv) ? Skv : kv_len;
+  int n_cu = 0;
+  dt::SplitPlan sp;
+  if (dt::plan_launch(B, Hq, Sq, kv_end, dt::kernel_dim(D), ~size_t(0), &n_cu,
+                      &sp) != DT_OK)
+    return 0;
+  return sp.ws_bytes;
 }
 
 extern "C" size_t dt_flash_fwd_workspace_bytes(int B, int Hq, int Sq, int Skv,

@@ -1,11 +1,15 @@
-// Flash attention forward for head dim 256 (gfx950): the head dims above
-// 128 that kernels/splash.py accepts (it requires only D_v % 8 == 0,
-// kernels/splash.py:156-160); dims 136..248 run zero-padded to 256 by the
-// Python layer, as the smaller dims pad to 64 or 128.  Same contract as
-// flash_attn_kernel (kernels/splash.py:566-650 and the residual form
-// :665-742): GQA, a host or device key length (one for the batch or one per
-// batch element), residual (o, m, l) outputs, the fixed-m operand.  Not
-// here: E4M3 keys, block-sparse tables, packed V and the tail split.
+// Flash attention forward for head dims 136 to 256 (gfx950): the head dims
+// above 128 that kernels/splash.py accepts (it requires only D_v % 8 == 0,
+// kernels/splash.py:156-160).  Same contract as flash_attn_kernel
+// (kernels/splash.py:566-650 and the residual form :665-742): GQA, a host or
+// device key length (one for the batch or one per batch element), residual
+// (o, m, l) outputs, the fixed-m operand, the tail split.  Not here: E4M3
+// keys, block-sparse tables and packed V.
+//
+// NB is the dim rounded up to 32 channels: NB output blocks and 2 NB QK
+// steps.  A dim below 256 is read and written as it is in memory; the LDS
+// rows keep 512 bytes, and the tile DMA fills the chunks past the dim with
+// zeros (their offset lies outside the descriptor's range).
 //
 // The D = 128 kernel's layout does not fit this width: two wavefronts per
 // SIMD leave 256 registers each, and Q^T (64) + O^T (128) + the scores do
@@ -39,6 +43,7 @@
 
 #include "../../include/dt_attention.h"
 #include "flash_common.h"
+#include "split_merge.h"
 
 namespace dt {
 namespace {
@@ -56,13 +61,11 @@ constexpr int kWVOff = kWStages * kWTileB;  // V stages after the K stages
 constexpr int kWLds = 2 * kWVOff;         // 128 KiB
 constexpr int kWLoads = kWTileB / 1024 / kWNW;  // 1 KiB DMAs per wave, K or V
 constexpr int kWGroup = 2 * kWLoads;      // DMA instructions per iteration
-constexpr int kWSteps = kWD / 16;         // QK channel steps
-constexpr int kWNB = kWD / 32;            // 32-channel output blocks
+constexpr int kWRead = 2;                 // operand reads ahead of their MFMA
 constexpr float kWTrip = 4096.0f;
 constexpr float kWShift = 24.0f;          // online heads' reference offset
 constexpr float kWTripShifted = kWTrip * 16777216.0f;  // 2^(12 + 24)
 constexpr float kWRecenter = 88.0f;       // kernels/fixed_m_bound.py:42
-static_assert(kWSteps == 16 && kWNB == 8, "one QK and one PV MFMA per slot");
 
 template <int N>
 using WStage = std::integral_constant<int, N>;
@@ -147,7 +150,10 @@ __device__ __forceinline__ void wide_mask(f32x16& s, int kv0, int hf,
   }
 }
 
+template <int NB>
 __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
+  constexpr int kWNB = NB;         // 32-channel output blocks
+  constexpr int kWSteps = 2 * NB;  // QK channel steps, one per PV MFMA
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds_raw[];
   lds_u8* lds = (lds_u8*)lds_raw;
   const int lane = threadIdx.x & 63;
@@ -155,7 +161,15 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
   const int l32 = lane & 31;
   const int hf = lane >> 5;
 
-  const int wg = xcd_remap(blockIdx.x, p.n_wg);
+  // tail split, as in flash_attn_kernel: unit >= 0 names (query block, part)
+  int wg, unit = -1, part = 0;
+  if ((int)blockIdx.x < p.n_main) {
+    wg = xcd_remap(blockIdx.x, p.n_main);
+  } else {
+    unit = blockIdx.x - p.n_main;
+    wg = p.n_main + unit / p.n_split;
+    part = unit - (unit / p.n_split) * p.n_split;
+  }
   const int qblk = wg % p.n_qblk;
   const int bh = wg / p.n_qblk;
   const int h = bh % p.Hq;
@@ -166,25 +180,60 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
   const uint16_t* vbase = p.v + b * p.v_sb + hk * p.v_sh;
   const int q0 = qblk * kWBQ + wave * 32;
   const int row = q0 + l32;  // this lane's query row
-  const int kv_end =
+  int kv_end =
       resolve_len(p.kv_len_dev, p.kv_len_count, b, p.kv_end, p.Skv);
-  const int ntiles = (kv_end + kWBKV - 1) / kWBKV;
+  int ntiles = (kv_end + kWBKV - 1) / kWBKV;
+  if (unit >= 0) {
+    // a split part's share of the tiles, as keys and values of its own
+    const int tbeg = (ntiles * part) / p.n_split;
+    ntiles = (ntiles * (part + 1)) / p.n_split - tbeg;
+    kbase += (int64_t)tbeg * kWBKV * p.k_ss;
+    vbase += (int64_t)tbeg * kWBKV * p.v_ss;
+    kv_end -= tbeg * kWBKV;
+    if (kv_end > ntiles * kWBKV) kv_end = ntiles * kWBKV;
+  }
+  const int dim = p.dim;
+  // outputs of row `row`: its own place, or the part's in the workspace (rows
+  // of 256 floats); worked out where they are used, so that they hold no
+  // registers during the sweep
+  struct Out {
+    float *o32, *m, *l;  // of this row, or nulls
+    uint16_t* o;
+  };
+  auto outputs = [&]() {
+    Out x{nullptr, nullptr, nullptr, nullptr};
+    if (unit >= 0) {
+      const int64_t units = (int64_t)p.n_tail * p.n_split;
+      const int64_t r = (int64_t)unit * kWBQ + (row - qblk * kWBQ);
+      x.o32 = p.ws + r * kWD;
+      x.m = p.ws + units * kWBQ * kWD + r;
+      x.l = x.m + units * kWBQ;
+      return x;
+    }
+    const int64_t r = ((int64_t)b * p.Hq + h) * p.Sq + row;
+    if (p.o32 != nullptr) {
+      x.o32 = p.o32 + r * dim;
+      x.m = p.m + r;
+      x.l = p.l + r;
+    }
+    if (p.o != nullptr)
+      x.o = p.o + b * p.o_sb + h * p.o_sh + (int64_t)row * p.o_ss;
+    return x;
+  };
 
   if (ntiles <= 0) {  // no keys (a device length of 0): the empty result
     if (row < p.Sq) {
-      const int64_t bhrow = ((int64_t)b * p.Hq + h) * p.Sq + row;
+      const Out x = outputs();
 #pragma unroll
       for (int j = 0; j < kWD / 8; ++j) {
-        if (p.o32 != nullptr)
-          *(u32x4*)(p.o32 + bhrow * kWD + (kWD / 2) * hf + 4 * j) =
-              u32x4{0u, 0u, 0u, 0u};
-        if (p.o != nullptr)
-          *(u32x2*)(p.o + b * p.o_sb + h * p.o_sh + (int64_t)row * p.o_ss +
-                    (kWD / 2) * hf + 4 * j) = u32x2{0u, 0u};
+        const int ch = (kWD / 2) * hf + 4 * j;
+        if (ch >= dim) continue;
+        if (x.o32 != nullptr) *(u32x4*)(x.o32 + ch) = u32x4{0u, 0u, 0u, 0u};
+        if (x.o != nullptr) *(u32x2*)(x.o + ch) = u32x2{0u, 0u};
       }
-      if (p.o32 != nullptr && hf == 0) {
-        p.m[bhrow] = 0.f;
-        p.l[bhrow] = 0.f;
+      if (x.o32 != nullptr && hf == 0) {
+        *x.m = 0.f;
+        *x.l = 0.f;
       }
     }
     return;
@@ -197,14 +246,16 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
   {
     const bool live = row < p.Sq;
     const uint16_t* qrow = qbase + (int64_t)(live ? row : p.Sq - 1) * p.q_ss;
-    const uint32_t keep = live ? 0xffffffffu : 0u;
     u32x4 raws[kWSteps];
 #pragma unroll
-    for (int t = 0; t < kWSteps; ++t)
-      raws[t] = *(const u32x4*)(qrow + 16 * t + 8 * hf);
+    for (int t = 0; t < kWSteps; ++t) {
+      const int ch = 16 * t + 8 * hf;
+      raws[t] = *(const u32x4*)(qrow + (ch < dim ? ch : 0));
+    }
 #pragma unroll
     for (int t = 0; t < kWSteps; ++t) {
       u32x4 r = raws[t];
+      const uint32_t keep = live && 16 * t + 8 * hf < dim ? 0xffffffffu : 0u;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const uint32_t w = r[e] & keep;
@@ -230,8 +281,9 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
   for (int i = 0; i < kWLoads; ++i) {
     const int r = wave * 8 + 2 * i + (lane >> 5);
     const int pc = lane & 31;
-    kvo[i] = r * krow + ((pc ^ (r & 15)) * 16);
-    vvo[i] = r * vrow + ((pc ^ (4 * (r & 3))) * 16);
+    const int kc = pc ^ (r & 15), vc = pc ^ (4 * (r & 3));
+    kvo[i] = 8 * kc < dim ? r * krow + kc * 16 : 0xffffff00u;
+    vvo[i] = 8 * vc < dim ? r * vrow + vc * 16 : 0xffffff00u;
   }
   const uint32_t lds_k = (uint32_t)(uintptr_t)lds + (uint32_t)wave * 8 * kWRow;
   const uint32_t lds_v = lds_k + kWVOff;
@@ -310,11 +362,12 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
         bf16x8, *(const __attribute__((address_space(3))) u32x4*)(
                     lds + kread[t & 7] + (S * kWTileB + 256 * (t >> 3))));
   };
-  // operand of PV MFMA i: key step i >> 3, output block i & 7
+  // operand of PV MFMA i: key step i / NB, output block i % NB
   auto vld = [&](auto stage, int i) {
     constexpr int S = decltype(stage)::value;
-    const lds_u8* a = lds + vread[i & 3] +
-                      (S * kWTileB + (i >> 3) * 16 * kWRow + 256 * ((i >> 2) & 1));
+    const int mb = i % NB;
+    const lds_u8* a = lds + vread[mb & 3] +
+                      (S * kWTileB + (i / NB) * 16 * kWRow + 256 * (mb >> 2));
     const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
         (__attribute__((address_space(3))) v4i16*)(a));
     const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
@@ -421,10 +474,10 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
   }
 
   // Iteration j (ring stage S = j % 4 of V, (j + 2) % 4 of K): on entry sc
-  // holds S(j+1) and pwc P(j).  32 MFMA slots alternate the QK product of
+  // holds S(j+1) and pwc P(j).  4 NB MFMA slots alternate the QK product of
   // tile j+2 (one accumulator chain into sn) with the PV product of tile j;
-  // beside each MFMA one VALU step of P(j+1) (two exps, a pack and a row-sum
-  // dot2 per pair of scores) into pwn.  Then the trip check of P(j+1), and
+  // spread over them the 32 VALU steps of P(j+1) (two exps, a pack and a
+  // row-sum dot2 per pair of scores) into pwn.  Then the trip check of P(j+1), and
   // the mask of tile j+2 if it is the last, partial one.  When j+2 is past
   // the last tile, QK runs on a zero-filled stage and its scores are never
   // used.
@@ -442,47 +495,60 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
     // order, waited behind its own with no MFMA running.
     const TileReq rk = req_k(j + kWKAhead), rv = req_v(j + kWVAhead);
     bf16x8 kr[4], vr[4];
-    kr[0] = kld(KS{}, 0);
-    vr[0] = vld(stage, 0);
-    kr[1] = kld(KS{}, 1);
-    vr[1] = vld(stage, 1);
-    float sa = 0.f, sb = 0.f, e0 = 0.f, e1 = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      if (i + 2 < 16) {
-        kr[(i + 2) & 3] = kld(KS{}, i + 2);
-        vr[(i + 2) & 3] = vld(stage, i + 2);
+    for (int i = 0; i < kWRead; ++i) {
+      kr[i] = kld(KS{}, i);
+      vr[i] = vld(stage, i);
+    }
+    float sa = 0.f, sb = 0.f, e0 = 0.f, e1 = 0.f;
+    // step st of the 32: pair st / 4 of the scores, its exps, pack, row sum
+    auto valu_step = [&](int st) {
+      const int q = st >> 2;
+      if ((st & 3) == 0) {
+        e0 = __builtin_amdgcn_exp2f(sc[2 * q]);
+        wpin(e0);
+      } else if ((st & 3) == 1) {
+        e1 = __builtin_amdgcn_exp2f(sc[2 * q + 1]);
+        wpin(e1);
+      } else if ((st & 3) == 2) {
+        pwn[q] = pack_bf16x2(e0, e1);
+        wpin(pwn[q]);
+      } else {
+        float& acc = (q & 1) ? sb : sa;
+        acc = dot2_acc(pwn[q], acc);
+        wpin(acc);
       }
-      const int q = i >> 1;
+    };
+#pragma unroll
+    for (int i = 0; i < kWSteps; ++i) {
+      if (i + kWRead < kWSteps) {
+        kr[(i + kWRead) & 3] = kld(KS{}, i + kWRead);
+        vr[(i + kWRead) & 3] = vld(stage, i + kWRead);
+      }
       if (i == 0)
         sn = qk_first(kr[0], qf[0], negm);
       else
         qk_acc(sn, kr[i & 3], qf[i]);
-      if (i & 1) {
-        pwn[q] = pack_bf16x2(e0, e1);
-        wpin(pwn[q]);
-        if (i < 8)
-          dma_k(rk, i >> 1);
-        else
-          dma_v(rv, (i - 8) >> 1);
-      } else {
-        e0 = __builtin_amdgcn_exp2f(sc[2 * q]);
-        wpin(e0);
-      }
+#pragma unroll
+      for (int st = 2 * i * 8 / NB; st < (2 * i + 1) * 8 / NB; ++st)
+        valu_step(st);
+#pragma unroll
+      for (int part = 0; part < kWGroup; ++part)
+        if (i == (2 * part + 1) * kWSteps / (2 * kWGroup)) {
+          if (part < kWLoads)
+            dma_k(rk, part);
+          else
+            dma_v(rv, part - kWLoads);
+        }
       __builtin_amdgcn_sched_barrier(0);
-      const int u = i >> 3, mb = i & 7;
+      const int u = i / NB, mb = i % NB;
       const u32x4 pr = {pwc[4 * u], pwc[4 * u + 1], pwc[4 * u + 2],
                         pwc[4 * u + 3]};
       o[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
           vr[i & 3], __builtin_bit_cast(bf16x8, pr), o[mb], 0, 0, 0);
-      if (i & 1) {
-        float& acc = (q & 1) ? sb : sa;
-        acc = dot2_acc(pwn[q], acc);
-        wpin(acc);
-      } else {
-        e1 = __builtin_amdgcn_exp2f(sc[2 * q + 1]);
-        wpin(e1);
-      }
+#pragma unroll
+      for (int st = (2 * i + 1) * 8 / NB; st < (2 * i + 2) * 8 / NB; ++st)
+        valu_step(st);
       __builtin_amdgcn_sched_barrier(0);
     }
     if (j + 1 < ntiles) settle(false, sc, pwn, sa + sb, sn);
@@ -512,36 +578,49 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
   if (row >= p.Sq) return;
   const float ltot = l + __shfl_xor(l, 32, 64);
   const float unshift = fixed ? 1.0f : 1.0f / 16777216.0f;  // 2^-kWShift
-  const int64_t bhrow = ((int64_t)b * p.Hq + h) * p.Sq + row;
-  if (p.o32 != nullptr) {
-    float* dst = p.o32 + bhrow * kWD;
+  const Out x = outputs();
+  if (x.o32 != nullptr) {
 #pragma unroll
     for (int mb = 0; mb < kWNB; ++mb)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
+        const int ch = 32 * mb + 8 * j + 4 * hf;
+        if (mb == kWNB - 1 && ch >= dim) continue;
         f32x4 w;
 #pragma unroll
         for (int e = 0; e < 4; ++e) w[e] = o[mb][4 * j + e] * unshift;
-        *(f32x4*)(dst + 32 * mb + 8 * j + 4 * hf) = w;
+        *(f32x4*)(x.o32 + ch) = w;
       }
     if (hf == 0) {
-      p.m[bhrow] = m + shift;
-      p.l[bhrow] = ltot * unshift;
+      *x.m = m + shift;
+      *x.l = ltot * unshift;
     }
   }
-  if (p.o != nullptr) {
+  if (x.o != nullptr) {
     const float inv = 1.0f / ltot;
-    uint16_t* dst = p.o + b * p.o_sb + h * p.o_sh + (int64_t)row * p.o_ss;
 #pragma unroll
     for (int mb = 0; mb < kWNB; ++mb)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
+        const int ch = 32 * mb + 8 * j + 4 * hf;
+        if (mb == kWNB - 1 && ch >= dim) continue;
         u32x2 w;
         w[0] = pack_bf16x2(o[mb][4 * j] * inv, o[mb][4 * j + 1] * inv);
         w[1] = pack_bf16x2(o[mb][4 * j + 2] * inv, o[mb][4 * j + 3] * inv);
-        *(u32x2*)(dst + 32 * mb + 8 * j + 4 * hf) = w;
+        *(u32x2*)(x.o + ch) = w;
       }
   }
+}
+
+template <int NB>
+int launch_wide(const FlashParams& p, hipStream_t st) {
+  static std::atomic<uint64_t> lds_set{0};
+  if (int rc = ensure_lds_limit((const void*)flash_wide_kernel<NB>, kWLds,
+                                lds_set, "dt_flash_fwd"))
+    return rc;
+  hipLaunchKernelGGL(flash_wide_kernel<NB>, dim3(p.n_main + p.n_tail * p.n_split),
+                     dim3(kWNW * 64), kWLds, st, p);
+  return DT_OK;
 }
 
 }  // namespace
@@ -556,21 +635,26 @@ int launch_flash_wide(const FlashParams& base, hipStream_t st) {
   const int64_t nwg = (int64_t)p.n_qblk * p.Hq * p.B;
   if (nwg > 0x7fffffff)
     return set_error(DT_ERR_SHAPE, "dt_flash_fwd: grid too large");
-  // byte offsets of one (b, h) slice's rows are 32-bit in the descriptors
-  if ((int64_t)p.kv_end * p.k_ss * 2 >= (1ll << 32) ||
-      (int64_t)p.kv_end * p.v_ss * 2 >= (1ll << 32))
+  // byte offsets of one (b, h) slice's rows are 32-bit in the descriptors (the
+  // chunks past a dim below 256 have one above them)
+  const int64_t range = (1ll << 32) - (p.dim < kWD ? 256 : 0);
+  if ((int64_t)p.kv_end * p.k_ss * 2 >= range ||
+      (int64_t)p.kv_end * p.v_ss * 2 >= range)
     return set_error(DT_ERR_SHAPE, "dt_flash_fwd: K/V slice above 4 GiB");
   p.n_wg = (int)nwg;
-  p.n_main = p.n_wg;
-  p.n_split = 1;
-  p.n_tail = 0;
-  p.ws = nullptr;
-  static std::atomic<uint64_t> lds_set{0};
-  if (int rc = ensure_lds_limit((const void*)flash_wide_kernel, kWLds, lds_set,
-                                "dt_flash_fwd"))
+  if (p.ws == nullptr || p.n_split <= 1) {
+    p.n_main = p.n_wg;
+    p.n_split = 1;
+    p.n_tail = 0;
+    p.ws = nullptr;
+  }
+  const int nb = (p.dim + 31) / 32;
+  if (int rc = nb <= 5   ? launch_wide<5>(p, st)
+               : nb == 6 ? launch_wide<6>(p, st)
+               : nb == 7 ? launch_wide<7>(p, st)
+                         : launch_wide<8>(p, st))
     return rc;
-  hipLaunchKernelGGL(flash_wide_kernel, dim3(p.n_wg), dim3(kWNW * 64), kWLds,
-                     st, p);
+  if (p.n_tail > 0) launch_split_merge<kWD, kWBQ>(p, st);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess)
     return set_error(DT_ERR_LAUNCH, "dt_flash_fwd: %s", hipGetErrorString(e));

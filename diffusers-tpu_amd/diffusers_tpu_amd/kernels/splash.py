@@ -27,10 +27,9 @@ Differences a caller can observe, all within the reference's tolerance:
   log2(e)`` is rounded to bf16 before the QK product (the kernel does this in
   registers with one rounding).
 * Head dims: the kernels are built for 64, 128 and 256.  Any other multiple
-  of 8 below 128 runs as it is (``dt_flash_fwd_anydim``); those from 136 to
-  248, and with ``qk_fp8`` every dim but 128, run zero-padded to the next of
-  them (zero channels change no score; the extra output channels are
-  dropped), with the scale of the real dim.  Above 256 (above 128 with ``qk_fp8``) raises
+  of 8 runs as it is in the next wider one (``dt_flash_fwd_anydim``); with
+  ``qk_fp8`` dims below 128 run zero-padded (zero channels change no score;
+  the extra output channels are dropped), with the scale of the real dim.  Above 256 (above 128 with ``qk_fp8``) raises
   ``NotImplementedError``, as does a dim that is not a multiple of 8
   (kernels/splash.py:156-160).
 * ``qk_fp8`` casts K to E4M3 in one GPU pass (``fp8_cast``) and the kernel
@@ -234,14 +233,14 @@ def _launch(query, key, value, scale, kv_len, out=None, residual=False,
                               "dims up to 256 (up to 128 with qk_fp8)")
   if not residual:
     _check_out(out, (b, hq, sq, d), query.device)
+  if (kd != d or d == 256) and not qk_fp8 and packed_v is None:
+    return _call_anydim(query, key, value, scale,
+                        n if n_dev is None else n_dev, out, residual, mk,
+                        workspace)
   if kd != d:
     if packed_v is not None:
       raise ValueError(f"packed_v is a head-dim-128 layout; head_dim={d} runs "
                        "zero-padded and packs its own V")
-    if d < 128 and not qk_fp8:
-      return _call_anydim(query, key, value, scale,
-                          n if n_dev is None else n_dev, out, residual, mk,
-                          workspace)
     # zero-padded channels: same scores, extra output channels dropped below
     res = _launch(pad_head_dim(query, kd), pad_head_dim(key, kd),
                   pad_head_dim(value, kd), scale,
@@ -314,7 +313,7 @@ def _call_anydim(query, key, value, scale, n, out, residual, mk, workspace):
                                          dtype=torch.bfloat16)
       outs = (o.data_ptr(), s3(o), None, None, None)
     nbytes = _split_bytes(b, hq, sq, skv, 0 if n_dev is not None else n_host,
-                          64 if d < 64 else 128, dev.index)
+                          d, dev.index)
     if not nbytes:
       ws = None
     elif workspace is not None:
@@ -333,9 +332,10 @@ def _call_anydim(query, key, value, scale, n, out, residual, mk, workspace):
 
 @functools.lru_cache(maxsize=4096)
 def _split_bytes(b, hq, sq, skv, n, d, device_index):
-  """``dt_flash_fwd_workspace_bytes`` per shape and device, queried once
-  (the current device is ``device_index`` when it is called)."""
-  return _lib.load().dt_flash_fwd_workspace_bytes(b, hq, sq, skv, n, d)
+  """``dt_flash_fwd_anydim_workspace_bytes`` (at head dims 64 and 128 the
+  bytes ``dt_flash_fwd_ex`` uses) per shape and device, queried once (the
+  current device is ``device_index`` when it is called)."""
+  return _lib.load().dt_flash_fwd_anydim_workspace_bytes(b, hq, sq, skv, n, d)
 
 
 def _call_ex(q, k, k_format, v, packed_v, out, residual, hkv, skv, scale, n,

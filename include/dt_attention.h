@@ -426,9 +426,9 @@ size_t dt_flash_fwd_workspace_bytes(int B, int Hq, int Sq, int Skv,
 
 /*
  * dt_flash_fwd_ex with bf16 keys, row-major V and no tile table, at any head
- * dim that is a multiple of 8 up to 128 (kernels/splash.py:156-160), and 256:
- * rows of D elements are read and written as they are, at the arithmetic of
- * the dim itself.  Rows of one (b, h) slice of q, k, v must not overlap
+ * dim that is a multiple of 8 up to 256 (kernels/splash.py:156-160): rows of
+ * D elements are read and written as they are, at the arithmetic of the dim
+ * itself, with the tail split at every dim.  Rows of one (b, h) slice of q, k, v must not overlap
  * (stride s >= D, or one row), and a K or V slice must span less than 4 GiB -
  * 256.  The default scale is 1/sqrt(D).
  */

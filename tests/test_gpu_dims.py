@@ -33,7 +33,7 @@ def _want(q, k, v, n=None, rows=None):
 
 
 @pytest.mark.parametrize("d", [8, 32, 40, 48, 56, 72, 80, 88, 96, 104, 112,
-                               120])
+                               120, 136, 160, 168, 192, 224, 248, 256])
 @pytest.mark.parametrize("shape", SHAPES, ids=[str(s) for s in SHAPES])
 def test_dim_matches_oracle(sp, d, shape):
   b, hq, hkv, sq, skv, n = shape
@@ -52,7 +52,7 @@ def test_dim_matches_oracle(sp, d, shape):
   assert torch.isfinite(o).all()
 
 
-@pytest.mark.parametrize("d", [40, 72, 112])
+@pytest.mark.parametrize("d", [40, 72, 112, 152])
 def test_views_and_outputs(sp, d):
   banner(f"dim {d}: views")
   b, h, s = 2, 3, 150
@@ -87,9 +87,10 @@ def test_views_and_outputs(sp, d):
   assert_attn_close(to64(v), want, "out is v")
 
 
-def test_fixed_m_and_device_lengths(sp):
-  banner("dim 88: fixed-m, device lengths")
-  q, k, v = (seeded((2, 4, 140, 88), 630 + i) for i in range(3))
+@pytest.mark.parametrize("d", [88, 200, 256])
+def test_fixed_m_and_device_lengths(sp, d):
+  banner(f"dim {d}: fixed-m, device lengths")
+  q, k, v = (seeded((2, 4, 140, d), 630 + i) for i in range(3))
   k = (k.float() - k.float().mean(dim=2, keepdim=True)).to(torch.bfloat16)
   got = sp.attention(q, k, v, use_fixed_m=True)
   assert_attn_close(to64(got), _want(q, k, v), "fixed-m")
