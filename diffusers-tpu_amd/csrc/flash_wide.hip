@@ -61,7 +61,7 @@ constexpr int kWVOff = kWStages * kWTileB;  // V stages after the K stages
 constexpr int kWLds = 2 * kWVOff;         // 128 KiB
 constexpr int kWLoads = kWTileB / 1024 / kWNW;  // 1 KiB DMAs per wave, K or V
 constexpr int kWGroup = 2 * kWLoads;      // DMA instructions per iteration
-constexpr int kWRead = 2;                 // operand reads ahead of their MFMA
+constexpr int kWRead = 3;                 // operand reads ahead of their MFMA
 constexpr float kWTrip = 4096.0f;
 constexpr float kWShift = 24.0f;          // online heads' reference offset
 constexpr float kWTripShifted = kWTrip * 16777216.0f;  // 2^(12 + 24)
@@ -429,6 +429,7 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
       l *= alpha;
 #pragma unroll
       for (int mb = 0; mb < kWNB; ++mb) scale_acc(o[mb], alpha);
+      mfma_drain();  // negm is read by the next QK chain, assembly as well
     }
     l += sum;
   };
@@ -474,32 +475,35 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
   }
 
   // Iteration j (ring stage S = j % 4 of V, (j + 2) % 4 of K): on entry sc
-  // holds S(j+1) and pwc P(j).  4 NB MFMA slots alternate the QK product of
-  // tile j+2 (one accumulator chain into sn) with the PV product of tile j;
-  // spread over them the 32 VALU steps of P(j+1) (two exps, a pack and a
-  // row-sum dot2 per pair of scores) into pwn.  Then the trip check of P(j+1), and
-  // the mask of tile j+2 if it is the last, partial one.  When j+2 is past
-  // the last tile, QK runs on a zero-filled stage and its scores are never
-  // used.
+  // holds S(j+1), pwc P(j), and kr, vr the first operands.  4 NB MFMA slots
+  // alternate the QK product of tile j+2 (one accumulator chain into sn) with
+  // the PV product of tile j; spread over them the 32 VALU steps of P(j+1)
+  // (two exps, a pack and a row-sum dot2 per pair of scores) into pwn.  Then
+  // the trip check of P(j+1), and the mask of tile j+2 if it is the last,
+  // partial one.  When j+2 is past the last tile, QK runs on a zero-filled
+  // stage and its scores are never used.
+  //
+  // The barrier stands in the middle of the iteration, where every wavefront
+  // has MFMAs on both sides of it, and the next iteration's first operands
+  // are read before this one's last MFMAs.  With the barrier between two
+  // iterations the matrix pipe ran empty from the last MFMA through the wait
+  // for the slowest wavefront, the drain of the score chain and the first
+  // operand reads (same box, B1 H8 S16384: dim 256 1985 -> 1871 us, dim 192
+  // 1613 -> 1593, dim 160 1456 -> 1450; reads 2 to 6 slots ahead ran alike).
+  bf16x8 kr[NB], vr[NB];
   auto iteration = [&](auto stage, int j, const f32x16& sc, f32x16& sn,
                        const uint32_t (&pwc)[8], uint32_t (&pwn)[8]) {
     constexpr int S = decltype(stage)::value;
     using KS = WStage<(S + 2) % kWStages>;
-    wait_vmcnt_c<2 * kWGroup>();  // K(j+2) and V(j) landed (this wave's part)
-    mfma_drain();                 // sc was written by the QK assembly
-    __syncthreads();              // ... and every wave's; iteration j-1 done
+    using KSNext = WStage<(S + 3) % kWStages>;
+    using VSNext = WStage<(S + 1) % kWStages>;
+    constexpr int kHalf = kWSteps / 2;
     // K(j+5) goes into the stage K(j+1) used, V(j+3) into the one V(j-1)
-    // used; their 8 DMA instructions are spread over the MFMA slots.  Issued
-    // together after the barrier, the 32 of the workgroup queued at the
+    // used; their 8 DMA instructions are spread over the MFMA slots behind
+    // the barrier.  Issued together, the 32 of the workgroup queued at the
     // CU's address unit for ~500 cycles, and each wavefront, issuing in
     // order, waited behind its own with no MFMA running.
     const TileReq rk = req_k(j + kWKAhead), rv = req_v(j + kWVAhead);
-    bf16x8 kr[4], vr[4];
-#pragma unroll
-    for (int i = 0; i < kWRead; ++i) {
-      kr[i] = kld(KS{}, i);
-      vr[i] = vld(stage, i);
-    }
     float sa = 0.f, sb = 0.f, e0 = 0.f, e1 = 0.f;
     // step st of the 32: pair st / 4 of the scores, its exps, pack, row sum
     auto valu_step = [&](int st) {
@@ -519,22 +523,43 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
         wpin(acc);
       }
     };
+    // the steps beside MFMA hs of the 4 NB: none beside the first (the score
+    // chain that sc came from is still draining), the others evenly
+    constexpr int kBeside = 2 * kWSteps - 1;
+    auto valu_beside = [&](int hs) {
+#pragma unroll
+      for (int st = hs == 0 ? 0 : (hs - 1) * 32 / kBeside;
+           st < (hs == 0 ? 0 : hs * 32 / kBeside); ++st)
+        valu_step(st);
+    };
 #pragma unroll
     for (int i = 0; i < kWSteps; ++i) {
-      if (i + kWRead < kWSteps) {
-        kr[(i + kWRead) & 3] = kld(KS{}, i + kWRead);
-        vr[(i + kWRead) & 3] = vld(stage, i + kWRead);
+      if (i == kHalf) {
+        // K(j+3) and V(j+1) landed (this wave's part, then every wave's), and
+        // every wave is done with iteration j-1's stages.  A bare barrier:
+        // the operand reads in flight are of stages nobody fills yet.
+        wait_vmcnt_c<kWGroup>();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      const int a = i + kWRead;  // operand read here: of the next iteration
+      if (a < kWSteps) {         // from its first on
+        kr[a % NB] = kld(KS{}, a);
+        vr[a % NB] = vld(stage, a);
+      } else {
+        kr[a % NB] = kld(KSNext{}, a - kWSteps);
+        vr[a % NB] = vld(VSNext{}, a - kWSteps);
       }
       if (i == 0)
         sn = qk_first(kr[0], qf[0], negm);
       else
-        qk_acc(sn, kr[i & 3], qf[i]);
-#pragma unroll
-      for (int st = 2 * i * 8 / NB; st < (2 * i + 1) * 8 / NB; ++st)
-        valu_step(st);
+        qk_acc(sn, kr[i % NB], qf[i]);
+      valu_beside(2 * i);
 #pragma unroll
       for (int part = 0; part < kWGroup; ++part)
-        if (i == (2 * part + 1) * kWSteps / (2 * kWGroup)) {
+        if (i == kHalf + part * kHalf / kWGroup) {
           if (part < kWLoads)
             dma_k(rk, part);
           else
@@ -545,10 +570,11 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
       const u32x4 pr = {pwc[4 * u], pwc[4 * u + 1], pwc[4 * u + 2],
                         pwc[4 * u + 3]};
       o[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-          vr[i & 3], __builtin_bit_cast(bf16x8, pr), o[mb], 0, 0, 0);
-#pragma unroll
-      for (int st = (2 * i + 1) * 8 / NB; st < (2 * i + 2) * 8 / NB; ++st)
-        valu_step(st);
+          vr[i % NB], __builtin_bit_cast(bf16x8, pr), o[mb], 0, 0, 0);
+      // the last QK MFMA of the iteration before has left the pipe three
+      // MFMAs ago, and its result's wait states are over here
+      if (i == 0) asm volatile("s_nop 7" ::: "memory");
+      valu_beside(2 * i + 1);
       __builtin_amdgcn_sched_barrier(0);
     }
     if (j + 1 < ntiles) settle(false, sc, pwn, sa + sb, sn);
@@ -558,6 +584,14 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
     }
   };
 
+  // K(2) and V(0) landed, and the first operands of iteration 0
+  wait_vmcnt_c<2 * kWGroup>();
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kWRead; ++i) {
+    kr[i] = kld(WStage<2>{}, i);
+    vr[i] = vld(WStage<0>{}, i);
+  }
   for (int j = 0;; j += 4) {
     iteration(WStage<0>{}, j, sA, sB, pwA, pwB);
     if (j + 1 >= ntiles) break;
