@@ -32,6 +32,7 @@
 #include <math.h>
 #include <stdint.h>
 #include <stdlib.h>
+#include <string.h>
 
 #include <type_traits>
 
@@ -511,6 +512,37 @@ int check_rot(int mode, int rot, int D) {
 namespace dt {
 namespace {
 
+// The frequency table of (axis_dims, theta).  A layer's calls repeat one
+// rotation, and its powers cost the host about as much as the launch: each
+// thread keeps the last table it made.
+void fill_freqs(NormRopeParams& p, const int32_t* axis_dims, float theta) {
+  struct Table {
+    int32_t dims[3] = {0, 0, 0};
+    float theta = 0.f;  // (0: none yet)
+    float freq_rev[64];
+    int8_t pair_axis[64];
+  };
+  static thread_local Table t;
+  if (t.theta != theta || memcmp(t.dims, axis_dims, sizeof(t.dims)) != 0) {
+    int j = 0;
+    for (int a = 0; a < 3; ++a) {
+      for (int i = 0; i < axis_dims[a] / 2; ++i, ++j) {
+        const double f = pow((double)theta, -2.0 * i / axis_dims[a]);
+        t.freq_rev[j] = (float)(f / (2.0 * M_PI));
+        t.pair_axis[j] = (int8_t)a;
+      }
+      t.dims[a] = axis_dims[a];
+    }
+    for (; j < 64; ++j) {
+      t.freq_rev[j] = 0.f;
+      t.pair_axis[j] = 0;
+    }
+    t.theta = theta;
+  }
+  memcpy(p.freq_rev, t.freq_rev, sizeof(t.freq_rev));
+  memcpy(p.pair_axis, t.pair_axis, sizeof(t.pair_axis));
+}
+
 // dt_qk_norm_rope and dt_qk_norm_rope_f32 (F32IN: fp32 q and k).
 template <bool F32IN>
 int norm_rope_entry(const void* q, const void* k,
@@ -541,14 +573,7 @@ int norm_rope_entry(const void* q, const void* k,
     if (int rc = check_rot(mode, rot, D)) return rc;
     p.rot = rot;
     p.pos = pos;
-    int j = 0;
-    for (int a = 0; a < 3; ++a) {
-      for (int i = 0; i < axis_dims[a] / 2; ++i, ++j) {
-        const double f = pow((double)theta, -2.0 * i / axis_dims[a]);
-        p.freq_rev[j] = (float)(f / (2.0 * M_PI));
-        p.pair_axis[j] = (int8_t)a;
-      }
-    }
+    fill_freqs(p, axis_dims, theta);
   }
   return launch_norm_rope<false, F32IN>(p, D, (hipStream_t)stream);
 }

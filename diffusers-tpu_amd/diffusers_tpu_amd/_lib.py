@@ -132,6 +132,39 @@ def strides3(strides: tuple) -> ctypes.Array:
   return i64_array(*strides[:3])
 
 
+@functools.lru_cache(maxsize=256)
+def i32_tuple(vals: tuple) -> ctypes.Array:
+  """``i32_array`` of a tuple, one shared read-only array per value."""
+  return i32_array(*vals)
+
+
+class _NoGuard:
+  def __enter__(self):
+    return None
+
+  def __exit__(self, *exc):
+    return False
+
+
+_NO_GUARD = _NoGuard()
+
+
+def device_guard(index: int):
+  """``torch.cuda.device(index)``, or nothing where ``index`` is the current
+  device already (entering torch's guard costs over a microsecond)."""
+  import torch
+  if torch.cuda.current_device() == index:
+    return _NO_GUARD
+  return torch.cuda.device(index)
+
+
+def raw_stream(index: int) -> int:
+  """The hipStream_t of torch's current stream on device ``index`` (without
+  the stream object ``torch.cuda.current_stream`` builds, about 2 us)."""
+  import torch
+  return torch._C._cuda_getCurrentRawStream(index)
+
+
 _host_lengths = {}
 
 

@@ -41,10 +41,10 @@ def quantize_saturating(x: torch.Tensor, *, factor: float = 1.0,
                      "with a contiguous last axis")
   b, h, s, d = x.shape
   lib = _lib.load()
-  with torch.cuda.device(x.device):
+  with _lib.device_guard(x.device.index):
     rc = lib.dt_quantize_e4m3(
         x.data_ptr(), out.data_ptr(), b, h, s, d,
         _lib.i64_array(*x.stride()[:3]), _lib.i64_array(*out.stride()[:3]),
-        float(factor), torch.cuda.current_stream(x.device).cuda_stream)
+        float(factor), _lib.raw_stream(x.device.index))
   _lib.check("dt_quantize_e4m3", rc)
   return out

@@ -71,7 +71,7 @@ def smooth_keys(key: torch.Tensor, kv_len=None, *, out=None,
     raise ValueError("out must be a bf16 (B, H, S, D) tensor on key's device "
                      "with a contiguous last axis and 8-element strides")
   lib = _lib.load()
-  with torch.cuda.device(key.device):
+  with _lib.device_guard(key.device.index):
     nbytes = lib.dt_smooth_keys_workspace_bytes(b, h, s, d,
                                                 0 if n_dev is not None else n)
     ws = torch.empty((nbytes + 3) // 4, device=key.device, dtype=torch.float32)
@@ -82,6 +82,6 @@ def smooth_keys(key: torch.Tensor, kv_len=None, *, out=None,
         _lib.i64_array(*key.stride()[:3]), _lib.i64_array(*out.stride()[:3]),
         n, _lib.ptr(n_dev), None if kn is None else kn.data_ptr(),
         ws.data_ptr(), nbytes,
-        torch.cuda.current_stream(key.device).cuda_stream)
+        _lib.raw_stream(key.device.index))
   _lib.check("dt_smooth_keys", rc)
   return (out, kn) if norms else out

@@ -99,7 +99,8 @@ def check_halves(cos, sin):
 
 def _table_operand(t, b, s, dev, name):
   """fp32 view (or copy) of a table and its (batch, seq) strides."""
-  t = t.to(device=dev, dtype=torch.float32)
+  if t.dtype is not torch.float32 or t.device != dev:
+    t = t.to(device=dev, dtype=torch.float32)
   if t.dim() == 2:
     t = t.unsqueeze(0)
   if t.dim() != 3 or t.shape[1] != s or t.shape[0] not in (1, b):
@@ -109,6 +110,13 @@ def _table_operand(t, b, s, dev, name):
     t = t.contiguous()
   sb = 0 if t.shape[0] == 1 else t.stride(0)
   return t, sb, t.stride(1)
+
+
+def _vector(t, dev):
+  """``t`` as contiguous float32 on ``dev`` (itself where it is that)."""
+  if t.dtype is torch.float32 and t.device == dev and t.is_contiguous():
+    return t
+  return t.to(device=dev, dtype=torch.float32).contiguous()
 
 
 def _prep(t, name, keep_f32=False):
@@ -121,8 +129,8 @@ def _prep(t, name, keep_f32=False):
     raise ValueError(f"{name} must be [B, S, H, D], got {tuple(t.shape)}")
   if t.dtype != torch.bfloat16 and not (keep_f32 and t.dtype == torch.float32):
     t = t.to(torch.bfloat16)
-  if t.stride(-1) != 1 or any(s % 8 for s in t.stride()[:3]) or \
-     t.data_ptr() % 16:
+  s0, s1, s2, s3 = t.stride()
+  if s3 != 1 or (s0 | s1 | s2) & 7 or t.data_ptr() & 15:
     t = t.contiguous()
   return t
 
@@ -167,13 +175,13 @@ def qk_norm_rope(q, k, wq, wk, *, eps=1e-6, rope=None, q_head_scale=None,
     q = q.contiguous()
   b, s, h, d = q.shape
   dev = q.device
-  wq = wq.to(device=dev, dtype=torch.float32).contiguous()
-  wk = wk.to(device=dev, dtype=torch.float32).contiguous()
+  wq = _vector(wq, dev)
+  wk = _vector(wk, dev)
   if wq.shape != (d,) or wk.shape != (d,):
     raise ValueError(f"norm weights must be ({d},)")
   hs = None
   if q_head_scale is not None:
-    hs = q_head_scale.to(device=dev, dtype=torch.float32).contiguous()
+    hs = _vector(q_head_scale, dev)
     if hs.shape != (h,):
       raise ValueError(f"q_head_scale must be ({h},)")
   if out_layout == "bhsd":
@@ -183,8 +191,8 @@ def qk_norm_rope(q, k, wq, wk, *, eps=1e-6, rope=None, q_head_scale=None,
   else:
     raise ValueError(f"out_layout {out_layout!r}")
   if out is None:
-    qo = torch.empty(shape, device=dev, dtype=torch.bfloat16)
-    ko = torch.empty(shape, device=dev, dtype=torch.bfloat16)
+    qo = q.new_empty(shape, dtype=torch.bfloat16)
+    ko = torch.empty_like(qo)
   else:
     qo, ko = out
     if qo.shape != shape or ko.shape != shape or qo.stride() != ko.stride():
@@ -202,7 +210,7 @@ def qk_norm_rope(q, k, wq, wk, *, eps=1e-6, rope=None, q_head_scale=None,
   else:
     vl, vl_dev = _lib.length_arg(valid_len, s, dev, "valid_len", batch=b)
   lib = _lib.load()
-  stream = torch.cuda.current_stream(dev).cuda_stream
+  stream = _lib.raw_stream(dev.index)
   if isinstance(rope, RopeTable):
     if rope.mode not in ("half", "pair"):
       raise ValueError(f"rope table mode {rope.mode!r}")
@@ -218,20 +226,20 @@ def qk_norm_rope(q, k, wq, wk, *, eps=1e-6, rope=None, q_head_scale=None,
       sb, ss = (0 if n == 1 else cos.stride(0)), cos.stride(1)
     rot = 2 * cos.shape[-1]
     fn = lib.dt_qk_norm_rope_table_f32 if f32 else lib.dt_qk_norm_rope_table
-    with torch.cuda.device(dev):
+    with _lib.device_guard(dev.index):
       rc = fn(
           q.data_ptr(), k.data_ptr(), qo.data_ptr(), ko.data_ptr(), b, s, h,
           d, _lib.strides3(q.stride()), _lib.strides3(ostr),
           wq.data_ptr(), wk.data_ptr(), float(eps),
           None if hs is None else hs.data_ptr(), _MODES[rope.mode],
-          cos.data_ptr(), sin.data_ptr(), _lib.i64_array(sb, ss), rot, vl,
+          cos.data_ptr(), sin.data_ptr(), _lib.strides3((sb, ss)), rot, vl,
           _lib.ptr(vl_dev), stream)
     _lib.check("dt_qk_norm_rope_table_f32" if f32 else
                "dt_qk_norm_rope_table", rc)
     return qo, ko
   mode = _lib.ROPE_NONE
   pos_ptr = None
-  dims = _lib.i32_array(0, 0, 0)
+  dims = (0, 0, 0)
   theta = 1.0
   if rope is not None:
     if rope.mode not in _MODES:
@@ -240,16 +248,19 @@ def qk_norm_rope(q, k, wq, wk, *, eps=1e-6, rope=None, q_head_scale=None,
     pos = rope.positions
     if pos.shape != (s, 3):
       raise ValueError(f"positions must be ({s}, 3), got {tuple(pos.shape)}")
-    pos = pos.to(device=dev, dtype=torch.int32).contiguous()
+    if (pos.dtype is not torch.int32 or pos.device != dev or
+        not pos.is_contiguous()):
+      pos = pos.to(device=dev, dtype=torch.int32).contiguous()
     pos_ptr = pos.data_ptr()
-    dims = _lib.i32_array(*rope.axis_dims)
+    dims = tuple(rope.axis_dims)
     theta = float(rope.theta)
   fn = lib.dt_qk_norm_rope_f32 if f32 else lib.dt_qk_norm_rope
-  with torch.cuda.device(dev):
+  with _lib.device_guard(dev.index):
     rc = fn(
         q.data_ptr(), k.data_ptr(), qo.data_ptr(), ko.data_ptr(), b, s, h, d,
         _lib.strides3(q.stride()), _lib.strides3(ostr), wq.data_ptr(),
         wk.data_ptr(), float(eps), None if hs is None else hs.data_ptr(),
-        mode, pos_ptr, dims, theta, vl, _lib.ptr(vl_dev), stream)
+        mode, pos_ptr, _lib.i32_tuple(dims), theta, vl, _lib.ptr(vl_dev),
+        stream)
   _lib.check("dt_qk_norm_rope_f32" if f32 else "dt_qk_norm_rope", rc)
   return qo, ko

@@ -70,8 +70,8 @@ def _as_bf16_rows(t):
   """bf16 with a contiguous last axis and 8-aligned strides."""
   if t.dtype != torch.bfloat16:
     t = t.to(torch.bfloat16)
-  if t.stride(-1) != 1 or any(s % 8 for s in t.stride()[:3]) or \
-     t.data_ptr() % 16:
+  s0, s1, s2, s3 = t.stride()
+  if s3 != 1 or (s0 | s1 | s2) & 7 or t.data_ptr() & 15:
     t = t.contiguous()
   return t
 
@@ -173,7 +173,7 @@ class AttentionWorkspace:
       packed = d == 128 and n >= PACKED_V_MIN_KEYS
     if packed:
       self.packed_v(packed_v_numel(b, hkv, n))
-    with torch.cuda.device(self.device):
+    with _lib.device_guard(self.device.index):
       nbytes = _lib.load().dt_flash_fwd_anydim_workspace_bytes(
           b, hq, sq, skv, 0 if n == skv else n, d)
     if nbytes:
@@ -200,12 +200,98 @@ def _check_workspace(workspace, device):
                      f"{device}")
 
 
+def _launch_plain(query, key, value, scale, kv_len, residual, workspace):
+  """``_launch`` of what a model's layer passes, in a few microseconds of host
+  time: bf16 tensors that the kernels take as they are, on the current device,
+  at head dim 64 or 128 with row-major V.  ``None`` for any other call, also
+  for a wrong one: ``_launch`` then converts, or says what is wrong.  (A small
+  call's time is the host's: 16.7 us of it in ``_launch``, 8.5 here, where the
+  launch itself takes 4 and the output's allocation 1.5.)"""
+  T = torch.Tensor
+  if not (type(query) is T and type(key) is T and type(value) is T):
+    return None
+  dt = torch.bfloat16
+  qshape, kshape = query.shape, key.shape
+  if (query.dtype is not dt or key.dtype is not dt or value.dtype is not dt or
+      len(qshape) != 4 or len(kshape) != 4 or value.shape != kshape):
+    return None
+  b, hq, sq, d = qshape
+  bk, hkv, skv, dk = kshape
+  if (bk != b or dk != d or (d != 128 and d != 64) or
+      not (b > 0 and hq > 0 and sq > 0 and hkv > 0 and skv > 0) or hq % hkv):
+    return None
+  dev = query.get_device()
+  if (dev < 0 or key.get_device() != dev or value.get_device() != dev or
+      torch.cuda.current_device() != dev):
+    return None
+  qst, kst, vst = query.stride(), key.stride(), value.stride()
+  qp, kp, vp = query.data_ptr(), key.data_ptr(), value.data_ptr()
+  if (qst[3] != 1 or kst[3] != 1 or vst[3] != 1 or (qp | kp | vp) & 15 or
+      (qst[0] | qst[1] | qst[2] | kst[0] | kst[1] | kst[2] | vst[0] | vst[1] |
+       vst[2]) & 7):
+    return None
+  len_ptr = None
+  if kv_len is None:
+    n = plan = skv
+  elif type(kv_len) is int:
+    if not 1 <= kv_len <= skv:
+      return None
+    n = plan = kv_len
+  else:
+    if (type(kv_len) is not T or kv_len.dtype is not torch.int32 or
+        kv_len.dim() != 1 or kv_len.get_device() != dev or
+        not kv_len.is_contiguous()):
+      return None
+    n = kv_len.numel()
+    if n != 1 and n != b:
+      return None
+    n = 0 if n == 1 else n  # the entry count beside a device length
+    len_ptr, plan = kv_len.data_ptr(), 0
+  if d == 128 and (plan or skv) >= PACKED_V_MIN_KEYS:
+    return None
+  scale = 1.0 / math.sqrt(d) if scale is None else float(scale)
+  if not scale > 0:
+    return None
+  nbytes = _split_bytes(b, hq, sq, skv, plan, d, dev)
+  ws_ptr = None
+  if workspace is not None:
+    if (type(workspace) is not AttentionWorkspace or
+        workspace.device.index != dev):
+      return None
+    if nbytes:
+      ws_ptr = workspace.split(nbytes).data_ptr()
+  elif nbytes:
+    ws = torch.empty((nbytes + 3) // 4, device=query.device,
+                     dtype=torch.float32)
+    ws_ptr = ws.data_ptr()
+  strides3 = _lib.strides3
+  if residual:
+    o = query.new_empty(qshape, dtype=torch.float32)
+    m = query.new_empty((b, hq, sq, 1), dtype=torch.float32)
+    l = torch.empty_like(m)
+    outs = (None, None, o.data_ptr(), m.data_ptr(), l.data_ptr())
+  else:
+    o = torch.empty_like(query, memory_format=torch.contiguous_format)
+    outs = (o.data_ptr(), strides3(o.stride()), None, None, None)
+  rc = _lib.load().dt_flash_fwd_ex(
+      qp, kp, 0, vp, strides3(vst), None, 0, outs[0], b, hq, hkv, sq, skv, d,
+      strides3(qst), strides3(kst), outs[1], scale, n, len_ptr, None, None,
+      None, outs[2], outs[3], outs[4], ws_ptr, nbytes, _lib.raw_stream(dev))
+  if rc:
+    _lib.check("dt_flash_fwd_ex", rc)
+  return (o, m, l) if residual else o
+
+
 def _launch(query, key, value, scale, kv_len, out=None, residual=False,
             mk=None, qk_fp8=False, packed_v=None, workspace=None):
   """One attention call through ``dt_flash_fwd_ex``.  ``packed_v``: V
   already packed by ``pack_v`` with the same kv_len (else V is packed here
   when the key count reaches ``PACKED_V_MIN_KEYS``, into ``workspace`` when
   given); ``workspace``: an ``AttentionWorkspace``."""
+  if out is None and mk is None and not qk_fp8 and packed_v is None:
+    res = _launch_plain(query, key, value, scale, kv_len, residual, workspace)
+    if res is not None:
+      return res
   for n, t in (("query", query), ("key", key), ("value", value)):
     _check_bhsd(n, t)
   _check_same_device(query.device, key=key, value=value)
@@ -298,7 +384,7 @@ def _call_anydim(query, key, value, scale, n, out, residual, mk, workspace):
   n_host = _lib.dev_count(n_dev) if n_dev is not None else int(n)
   s3 = lambda t: _lib.strides3(t.stride())
   lib = _lib.load()
-  with torch.cuda.device(dev):
+  with _lib.device_guard(dev.index):
     if residual:
       o = torch.empty((b, hq, sq, d), device=dev, dtype=torch.float32)
       m = torch.empty((b, hq, sq, 1), device=dev, dtype=torch.float32)
@@ -324,7 +410,7 @@ def _call_anydim(query, key, value, scale, n, out, residual, mk, workspace):
         q.data_ptr(), k.data_ptr(), v.data_ptr(), outs[0], b, hq, hkv, sq, skv,
         d, s3(q), s3(k), s3(v), outs[1], scale, n_host, _lib.ptr(n_dev),
         _lib.ptr(mk), *outs[2:], _lib.ptr(ws), nbytes,
-        torch.cuda.current_stream(dev).cuda_stream))
+        _lib.raw_stream(dev.index)))
   if residual:
     return o, m, l
   return o if out is None else out if direct else out.copy_(o)
@@ -347,12 +433,12 @@ def _call_ex(q, k, k_format, v, packed_v, out, residual, hkv, skv, scale, n,
   b, hq, sq, d = q.shape
   _check_workspace(workspace, q.device)
   lib = _lib.load()
-  stream = torch.cuda.current_stream(q.device).cuda_stream
+  stream = _lib.raw_stream(q.device.index)
   s3 = lambda t: _lib.strides3(t.stride())
   n_dev = n if isinstance(n, torch.Tensor) else None
   # with a device length the host argument is its entry count
   n_host = _lib.dev_count(n_dev) if n_dev is not None else int(n)
-  with torch.cuda.device(q.device):
+  with _lib.device_guard(q.device.index):
     if residual:
       o = None
       o32 = torch.empty((b, hq, sq, d), device=q.device, dtype=torch.float32)
@@ -420,11 +506,11 @@ def pack_v(value, kv_len=None, out=None):
         vt.numel() < size or not vt.is_contiguous()):
       raise ValueError(f"out must be a contiguous bf16 tensor of at least "
                        f"{size} elements on value's device")
-  with torch.cuda.device(value.device):
+  with _lib.device_guard(value.device.index):
     rc = _lib.load().dt_pack_v(
         value.data_ptr(), vt.data_ptr(), b, hkv, skv, d,
         _lib.i64_array(*value.stride()[:3]), n, _lib.ptr(n_dev), tiles,
-        torch.cuda.current_stream(value.device).cuda_stream)
+        _lib.raw_stream(value.device.index))
   _lib.check("dt_pack_v", rc)
   return vt, tiles
 
@@ -580,10 +666,10 @@ def merge_residuals(parts):
     out = torch.empty_like(o)
     ptrs = [(ctypes.c_void_p * len(parts))(*(p[i].data_ptr() for p in parts))
             for i in range(3)]
-    with torch.cuda.device(o.device):
+    with _lib.device_guard(o.device.index):
       rc = _lib.load().dt_merge_residuals(
           *ptrs, len(parts), o.numel() // o.shape[-1], o.shape[-1],
-          out.data_ptr(), torch.cuda.current_stream(o.device).cuda_stream)
+          out.data_ptr(), _lib.raw_stream(o.device.index))
     _lib.check("dt_merge_residuals", rc)
     return out
   ms = torch.stack([p[1] for p in parts])
