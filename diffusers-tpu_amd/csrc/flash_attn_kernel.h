@@ -486,27 +486,29 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
     u32x4 rsrc;
     uint32_t lds;
   };
-  auto tile_rows = [&](bool valid, int kt) {
-    int rows = kv_end - kt * kBKV < kBKV ? kv_end - kt * kBKV : kBKV;
+  struct TileReqs {
+    TileReq k, v;
+  };
+  // both requests of one tile (the descriptors share its row count)
+  auto tile_reqs = [&](bool valid, int t, int kt) {
+    const int kv0 = kt * kBKV;
+    int rows = kv_end - kv0 < kBKV ? kv_end - kv0 : kBKV;
     // a listed tile may start past kv_end; readfirstlane keeps the clamp,
     // which the compiler forms as a vector med3, out of the scalar descriptor
     if constexpr (SPARSE) rows = __builtin_amdgcn_readfirstlane(rows < 0 ? 0 : rows);
-    return valid ? (uint32_t)rows : 0u;
-  };
-  auto req_k = [&](bool valid, int t, int kt) {
-    return TileReq{make_rsrc((uint64_t)(uintptr_t)kbase +
-                                 (uint64_t)(kt * kBKV) * krow,
-                             tile_rows(valid, kt) * krow),
-                   lds_k + (uint32_t)(t % kNStage) * L::kKTileB};
-  };
-  auto req_v = [&](bool valid, int t, int kt) {
+    if (!valid) rows = 0;
+    TileReqs r;
+    r.k.rsrc = make_rsrc((uint64_t)(uintptr_t)kbase + (uint64_t)kv0 * krow,
+                         (uint32_t)rows * krow);
     // a packed V tile is one contiguous 16 KiB block, zero past kv_end
-    return TileReq{
+    r.v.rsrc =
         VT ? make_rsrc((uint64_t)(uintptr_t)vbase + (uint64_t)kt * L::kVTileB,
                        valid ? (uint32_t)L::kVTileB : 0u)
-           : make_rsrc((uint64_t)(uintptr_t)vbase + (uint64_t)(kt * kBKV) * vrow,
-                       tile_rows(valid, kt) * vrow),
-        lds_v + (uint32_t)(t % kNStage) * L::kVTileB};
+           : make_rsrc((uint64_t)(uintptr_t)vbase + (uint64_t)kv0 * vrow,
+                       (uint32_t)rows * vrow);
+    r.k.lds = lds_k + (uint32_t)(t % kNStage) * L::kKTileB;
+    r.v.lds = lds_v + (uint32_t)(t % kNStage) * L::kVTileB;
+    return r;
   };
   auto dma_k = [&](const TileReq& r, int i) {
     lds_dma16_buf(r.rsrc, kvo[i], r.lds + i * 1024);
@@ -517,19 +519,19 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
   // DMA instruction `part` of an iteration's requests: the K parts first (K
   // is read one phase earlier than V: 0.25-0.45 % at V7 against interleaving
   // the two)
-  auto dma_part = [&](const TileReq& rk, const TileReq& rv, int part) {
+  auto dma_part = [&](const TileReqs& r, int part) {
     if (part < L::kKLoads)
-      dma_k(rk, part);
+      dma_k(r.k, part);
     else
-      dma_v(rv, part - L::kKLoads);
+      dma_v(r.v, part - L::kKLoads);
   };
   auto issue_k = [&](int t) {
-    const TileReq r = req_k(t < ntiles, t, t < ntiles ? tile_of(t) : 0);
+    const TileReq r = tile_reqs(t < ntiles, t, t < ntiles ? tile_of(t) : 0).k;
 #pragma unroll
     for (int i = 0; i < L::kKLoads; ++i) dma_k(r, i);
   };
   auto issue_v = [&](int t) {
-    const TileReq r = req_v(t < ntiles, t, t < ntiles ? tile_of(t) : 0);
+    const TileReq r = tile_reqs(t < ntiles, t, t < ntiles ? tile_of(t) : 0).v;
 #pragma unroll
     for (int i = 0; i < L::kVLoads; ++i) dma_v(r, i);
   };
@@ -809,15 +811,14 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
     // the interleaved phase; the epilogue drains it).  Of 4 wavefronts, K of
     // tile jt+2 goes into the stage of K(jt), whose scores are done, and V
     // of tile jt+1 into the stage of V(jt-1).
-    const TileReq rk = req_k(jt + kDist < ntiles, jt + kDist, t_issue);
-    const TileReq rv =
-        R == 8 ? req_v(jt + kDist < ntiles, jt + kDist, t_issue)
-                : req_v(has_next, jt + 1, k_next / kBKV);  // (k_next: tile jt+1)
+    TileReqs req = tile_reqs(jt + kDist < ntiles, jt + kDist, t_issue);
+    if constexpr (R != 8)  // (k_next: tile jt+1)
+      req.v = tile_reqs(has_next, jt + 1, k_next / kBKV).v;
     constexpr int NM = QK8 ? 4 : 2 * L::kSteps, NP = L::kLoadsPerTile;
     auto dma = [&](int i) {
 #pragma unroll
       for (int part = 0; part < NP; ++part)
-        if (i == (2 * part + 1) * NM / (2 * NP)) dma_part(rk, rv, part);
+        if (i == (2 * part + 1) * NM / (2 * NP)) dma_part(req, part);
     };
     // second half of tile jt (first half already in pw, its sum in hsum)
     // (On the last tile the QK product runs on a stale or zero-filled LDS
