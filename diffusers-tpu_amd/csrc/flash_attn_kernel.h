@@ -249,6 +249,9 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
   constexpr int NB = L::kNB;
   constexpr int kNStage = L::kNStage;
   constexpr int kRowsPerWave = L::kRowsPerWave;
+  // q rows through LDS (see q_dma below)
+  constexpr bool kQDma = R == 4 && G == 1;
+  constexpr int kQRowsB = 32 * 2 * D;  // bytes of a wavefront's q rows
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds_raw[];
   lds_u8* lds = (lds_u8*)lds_raw;
 
@@ -366,7 +369,7 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
   // of its row for step t, one byte each, in channel order.
   bf16x8 qf[L::kSteps];
   i32x8 qf8[2];
-  {
+  auto load_q = [&]() {
     // Rows past Sq load row Sq-1 (in bounds) and are zeroed after: loads
     // under a per-row branch were issued in two dependent batches (the
     // compiler waited for the first two before issuing the rest), one
@@ -414,7 +417,8 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
           }
         }
     }
-  }
+  };
+  if constexpr (!kQDma) load_q();
 
   // ---- tile loads: wave w fills rows 8w .. 8w+7 (of 4 wavefronts: 16w ..
   // 16w+15) of the K and V tiles;
@@ -534,6 +538,55 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
     const TileReq r = tile_reqs(t < ntiles, t, t < ntiles ? tile_of(t) : 0).v;
 #pragma unroll
     for (int i = 0; i < L::kVLoads; ++i) dma_v(r, i);
+  };
+
+  // With few tiles per block the q rows are a large part of what a workgroup
+  // reads.  Loaded straight into the operand layout an instruction takes 32
+  // bytes of 32 rows, and the line of a row is asked for four times, by when
+  // the CU's L1 has often lost it; here each wavefront brings its 32 rows by
+  // whole lines (as a K tile's, same swizzle) into LDS that is free until
+  // V(1) is requested, and reads its operands from there.  H40 Sq 48360, with
+  // the output stored past the caches (p.nt_out) on both sides: Skv 64 237 ->
+  // 231 us, 256 387 -> 372, 512 582 -> 570; D = 64, Skv 64 145 -> 135.
+  // (Direct loads with the non-temporal hint, which gives a line up at once:
+  // 317 us at Skv 64.)
+  const int q_region = (wave < 2 ? L::kLds + wave * kQRowsB
+                                 : L::kVOff + L::kVTileB + (wave - 2) * kQRowsB);
+  auto q_dma = [&]() {
+    constexpr int NCH = 2 * D / 16, RPI = 64 / NCH;
+    int rows = p.Sq - q0;
+    rows = __builtin_amdgcn_readfirstlane(rows < 0 ? 0 : (rows < 32 ? rows : 32));
+    const uint32_t qrow = (uint32_t)p.q_ss * 2u;
+    const u32x4 rsrc =
+        make_rsrc((uint64_t)(uintptr_t)qbase + (uint64_t)(rows > 0 ? q0 : 0) * qrow,
+                  (uint32_t)rows * qrow);
+#pragma unroll
+    for (int i = 0; i < 32 / RPI; ++i) {
+      const int row = i * RPI + lane / NCH;
+      const int ch = (lane % NCH) ^ (D == 128 ? row & 15 : (row >> 1) & 7);
+      lds_dma16_buf(rsrc, chunk_at(row * qrow, ch),
+                    (uint32_t)(uintptr_t)lds + q_region + i * 1024);
+    }
+  };
+  auto q_from_lds = [&]() {
+    // the tiles requested behind them may stay in flight
+    wait_vmcnt_c<2 * L::kKLoads + L::kVLoads>();
+    asm volatile("" ::: "memory");
+    u32x4 raws[L::kSteps];
+#pragma unroll
+    for (int t = 0; t < L::kSteps; ++t)
+      raws[t] = *(const __attribute__((address_space(3))) u32x4*)(
+          lds + q_region + l32 * (2 * D) +
+          ((2 * t + hf) ^ (D == 128 ? l32 & 15 : (l32 >> 1) & 7)) * 16);
+#pragma unroll
+    for (int t = 0; t < L::kSteps; ++t) {
+      u32x4 raw = raws[t];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        raw[e] = pack_bf16x2(__uint_as_float(raw[e] << 16) * c,
+                             __uint_as_float(raw[e] & 0xffff0000u) * c);
+      qf[t] = __builtin_bit_cast(bf16x8, raw);
+    }
   };
 
   // ---- per-lane LDS operand offsets (bytes within a stage, plus the key
@@ -771,9 +824,21 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
     }
     wait_vmcnt_c<L::kLoadsPerTile>();  // tile 0 landed
   } else {
+    bool via_lds = false;
+    if constexpr (kQDma) {
+      // (rows that overlap or lie far apart are read directly)
+      via_lds = p.q_ss >= dim && p.q_ss < (1 << 24);
+      if (via_lds) q_dma();
+    }
     issue_k(0);
     issue_v(0);
     issue_k(1);
+    if constexpr (kQDma) {
+      if (via_lds)
+        q_from_lds();
+      else
+        load_q();
+    }
     wait_vmcnt_c<L::kLoadsPerTile>();  // K(0) landed
   }
   __syncthreads();
@@ -998,7 +1063,9 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
         const u32x4 v = *slice_ptr(r);
         if (q0 + r < p.Sq && (!HD::RAGGED || ps * (RB / 2) + 8 * ck < dim)) {
           uint16_t* dst = obase + (int64_t)(q0 + r) * p.o_ss + ps * (RB / 2) + 8 * ck;
-          if (al16) {
+          if (al16 && p.nt_out) {
+            __builtin_nontemporal_store(v, (u32x4*)dst);
+          } else if (al16) {
             *(u32x4*)dst = v;
           } else {
             *(u32x2*)dst = u32x2{v[0], v[1]};
@@ -1015,6 +1082,8 @@ int launch_flash(const FlashParams& base, hipStream_t st) {
   constexpr int D = HD::D;
   using L = Stage<HD, QK8, R>;
   constexpr int BQ = R * 32;
+  // (4 x 1: room for the q rows of two wavefronts behind the ring)
+  constexpr int kLdsBytes = G * L::kLds + (R == 4 && G == 1 ? 2 * 32 * 2 * D : 0);
   FlashParams p = base;
   p.n_qblk = (p.Sq + BQ - 1) / BQ;
   const int64_t nwg = (int64_t)p.n_qblk * p.Hq * p.B;
@@ -1038,11 +1107,11 @@ int launch_flash(const FlashParams& base, hipStream_t st) {
   }
   const void* fn = (const void*)flash_attn_kernel<HD, QK8, SPARSE, VT, R, G>;
   static std::atomic<uint64_t> lds_set{0};
-  if (int rc = ensure_lds_limit(fn, G * L::kLds, lds_set, "dt_flash_fwd"))
+  if (int rc = ensure_lds_limit(fn, kLdsBytes, lds_set, "dt_flash_fwd"))
     return rc;
   const int grid = p.n_main + p.n_tail * p.n_split;
   hipLaunchKernelGGL((flash_attn_kernel<HD, QK8, SPARSE, VT, R, G>), dim3(grid),
-                     dim3(R * G * 64), G * L::kLds, st, p);
+                     dim3(R * G * 64), kLdsBytes, st, p);
   if (p.n_tail > 0) launch_split_merge<D, BQ>(p, st);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess)

@@ -49,6 +49,11 @@ struct FlashParams {
   // merge rounds as the tail split does; the entry points without a
   // workspace argument keep one order of tiles)
   bool key_groups;
+  // o is stored past the caches: more than half of the 256 MB Infinity Cache,
+  // it would only push out the K and V that the sweeps share (H40 Sq 48360
+  // D = 64, 248 MB: Skv 128 196 -> 169 us, 512 357 -> 336; D = 128, 495 MB:
+  // 586 -> 582; at 51 and 102 MB, and for long sweeps, no difference)
+  bool nt_out;
   int64_t q_sb, q_sh, q_ss;
   int64_t k_sb, k_sh, k_ss;
   int64_t v_sb, v_sh, v_ss;

@@ -177,6 +177,7 @@ int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
   p.n_tail = 0;
   p.n_main = 0;
   p.key_groups = key_groups;
+  p.nt_out = (int64_t)B * Hq * Sq * D * 2 > (128ll << 20);
   // (dt_flash_fwd_ex runs head dim 256 unsplit: the workspace is not used)
   if (ws != nullptr && (D != 256 || any_dim)) {
     if (!al16(ws))

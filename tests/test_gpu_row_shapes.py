@@ -64,3 +64,26 @@ def test_row_shapes_match_oracle(dta, case):
     shift = 2.0**-9 * np.einsum("bhid,bhjd->bhij", np.abs(c * q64),
                                 np.abs(kr)).max(-1)[..., None]
     assert (np.abs(lse - (wm + np.log2(wl))) <= shift + 2.0**-8).all()
+
+
+@pytest.mark.parametrize("d", [64, 72, 128])
+def test_queries_read_as_they_lie(dta, d):
+  """128-row workgroups bring their q rows in by DMA: rows with gaps and the
+  last, partial block; rows that overlap or repeat are read directly."""
+  banner(f"q rows at dim {d}")
+  h, sq, skv = 40, 700, 130
+  k = seeded((1, h, skv, d), 641)
+  v = seeded((1, h, skv, d), 642)
+  wide = seeded((1, sq, h, d + 8), 643)
+  flat = seeded((1, h, 8 * sq + d), 644)
+  views = {
+      "gaps": wide[..., :d].transpose(1, 2),
+      "overlapping": flat.unfold(2, d, 8)[:, :, :sq],
+      "one row": flat[:, :, :d].unsqueeze(2).expand(-1, -1, sq, -1),
+  }
+  wide[..., d:] = float("nan")
+  for name, q in views.items():
+    got = dta.attention(q, k, v)
+    rows = np.r_[0:3, 125:131, 255:258, sq - 70:sq]
+    want = A.attention_f64(to64(q[:, :, rows]), to64(k), to64(v))
+    assert_attn_close(to64(got[:, :, rows]), want, name)
