@@ -482,62 +482,93 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
   // (a packed V tile's wave share of 128-byte rows is as many bytes)
   const uint32_t lds_v = (uint32_t)(uintptr_t)lds + (uint32_t)grp * L::kLds + L::kVOff +
                          (uint32_t)wave * (kRowsPerWave * L::kVRow);
-  // One tile's request, K or V: its descriptor and LDS stage, for visit
-  // position t (which selects the stage) and key tile kt.  An invalid
-  // request (past the last tile) has an empty range: its DMAs read nothing
-  // and fill their stage with zeros.
-  struct TileReq {
+  // The requests.  With bf16 K, row-major V and no tile table, K and V are each
+  // a stream of tiles: the descriptor of the next one to request, which reaches
+  // from its first row to the end of the sweep and is advanced by a tile per
+  // request.  (Rebuilt from the tile's number it took 20 scalar instructions
+  // more per tile; without them B1 H24 S16896 D128 2613 -> 2581 us, B2 H24
+  // S4608 412.5 -> 407.3, B1 H8 S66868 D64 8158 -> 8062, B2 H16 S4096 D72
+  // 159.8 -> 156.2.)  Past the last tile nothing is left: the DMAs read
+  // nothing and fill their stage with zeros.  Listed tiles, packed V and E4M3
+  // K build the descriptors of their tile: at the power limit of the long
+  // sweeps that packed V serves the scalar instructions cost nothing (B1 H40
+  // S48872 37.71 ms, and 37.85 with streams), and E4M3 measured 2189 us against
+  // 2199 (H24 S16896).  Packed V has one contiguous 16 KiB block per tile, zero
+  // past kv_end.
+  constexpr bool kStream = !SPARSE && !VT && !QK8;
+  struct Stream {
+    uint64_t base;
+    uint32_t left;  // bytes (under 4 GiB by the check at the launch)
     u32x4 rsrc;
-    uint32_t lds;
   };
-  struct TileReqs {
-    TileReq k, v;
+  Stream ks, vs;
+  if constexpr (kStream) {
+    const int first_row = (tbeg + grp) * kBKV;
+    const int part_end = (tbeg + ntiles) * kBKV;
+    const int end_row = unit >= 0 && part_end < kv_end ? part_end : kv_end;
+    const uint32_t rows_left =
+        __builtin_amdgcn_readfirstlane(end_row > first_row ? end_row - first_row : 0);
+    ks.base = (uint64_t)(uintptr_t)kbase + (uint64_t)first_row * krow;
+    vs.base = (uint64_t)(uintptr_t)vbase + (uint64_t)first_row * vrow;
+    ks.left = rows_left * krow;
+    vs.left = rows_left * vrow;
+  }
+  auto advance = [&](Stream& s, uint32_t row) {
+    // (32 bits: a step that leaves bytes to read stays within the head's slice)
+    const uint32_t step = G * kBKV * row;
+    // (laundered: the compiler otherwise forms a vector saturating subtract,
+    // and the descriptor with it)
+    uint32_t n = s.left < step ? s.left : step;
+    asm("" : "+s"(n));
+    s.left -= n;
+    s.base += step;
   };
-  // both requests of one tile (the descriptors share its row count)
-  auto tile_reqs = [&](bool valid, int t, int kt) {
-    const int kv0 = kt * kBKV;
-    int rows = kv_end - kv0 < kBKV ? kv_end - kv0 : kBKV;
-    // a listed tile may start past kv_end; readfirstlane keeps the clamp,
-    // which the compiler forms as a vector med3, out of the scalar descriptor
+  // rows of tile kt: a listed tile may start past kv_end; readfirstlane keeps
+  // the clamp, which the compiler forms as a vector med3, out of the scalar
+  // descriptor
+  auto tile_rows = [&](bool valid, int kt) -> uint32_t {
+    int rows = kv_end - kt * kBKV < kBKV ? kv_end - kt * kBKV : kBKV;
     if constexpr (SPARSE) rows = __builtin_amdgcn_readfirstlane(rows < 0 ? 0 : rows);
-    if (!valid) rows = 0;
-    TileReqs r;
-    r.k.rsrc = make_rsrc((uint64_t)(uintptr_t)kbase + (uint64_t)kv0 * krow,
-                         (uint32_t)rows * krow);
-    // a packed V tile is one contiguous 16 KiB block, zero past kv_end
-    r.v.rsrc =
-        VT ? make_rsrc((uint64_t)(uintptr_t)vbase + (uint64_t)kt * L::kVTileB,
-                       valid ? (uint32_t)L::kVTileB : 0u)
-           : make_rsrc((uint64_t)(uintptr_t)vbase + (uint64_t)kv0 * vrow,
-                       (uint32_t)rows * vrow);
-    r.k.lds = lds_k + (uint32_t)(t % kNStage) * L::kKTileB;
-    r.v.lds = lds_v + (uint32_t)(t % kNStage) * L::kVTileB;
-    return r;
+    return valid ? rows : 0;
   };
-  auto dma_k = [&](const TileReq& r, int i) {
-    lds_dma16_buf(r.rsrc, kvo[i], r.lds + i * 1024);
+  // (valid: whether there is such a tile; kt: which)
+  auto next_k = [&](bool valid, int kt) {
+    if constexpr (kStream) {
+      ks.rsrc = make_rsrc(ks.base, ks.left);
+      advance(ks, krow);
+    } else {
+      ks.rsrc = make_rsrc((uint64_t)(uintptr_t)kbase + (uint64_t)(kt * kBKV) * krow,
+                          tile_rows(valid, kt) * krow);
+    }
   };
-  auto dma_v = [&](const TileReq& r, int i) {
-    lds_dma16_buf(r.rsrc, vvo[i], r.lds + i * 1024);
+  auto next_v = [&](bool valid, int kt) {
+    if constexpr (kStream) {
+      vs.rsrc = make_rsrc(vs.base, vs.left);
+      advance(vs, vrow);
+    } else {
+      vs.rsrc =
+          VT ? make_rsrc((uint64_t)(uintptr_t)vbase + (uint64_t)kt * L::kVTileB,
+                         valid ? (uint32_t)L::kVTileB : 0u)
+             : make_rsrc((uint64_t)(uintptr_t)vbase + (uint64_t)(kt * kBKV) * vrow,
+                         tile_rows(valid, kt) * vrow);
+    }
   };
-  // DMA instruction `part` of an iteration's requests: the K parts first (K
-  // is read one phase earlier than V: 0.25-0.45 % at V7 against interleaving
-  // the two)
-  auto dma_part = [&](const TileReqs& r, int part) {
-    if (part < L::kKLoads)
-      dma_k(r.k, part);
-    else
-      dma_v(r.v, part - L::kKLoads);
+  // DMA i of the wave's share of a tile, into ring stage `stage`
+  auto dma_k = [&](int stage, int i) {
+    lds_dma16_buf(ks.rsrc, kvo[i], lds_k + (uint32_t)(stage * L::kKTileB + i * 1024));
+  };
+  auto dma_v = [&](int stage, int i) {
+    lds_dma16_buf(vs.rsrc, vvo[i], lds_v + (uint32_t)(stage * L::kVTileB + i * 1024));
   };
   auto issue_k = [&](int t) {
-    const TileReq r = tile_reqs(t < ntiles, t, t < ntiles ? tile_of(t) : 0).k;
+    next_k(t < ntiles, !kStream && t < ntiles ? tile_of(t) : 0);
 #pragma unroll
-    for (int i = 0; i < L::kKLoads; ++i) dma_k(r, i);
+    for (int i = 0; i < L::kKLoads; ++i) dma_k(t % kNStage, i);
   };
   auto issue_v = [&](int t) {
-    const TileReq r = tile_reqs(t < ntiles, t, t < ntiles ? tile_of(t) : 0).v;
+    next_v(t < ntiles, !kStream && t < ntiles ? tile_of(t) : 0);
 #pragma unroll
-    for (int i = 0; i < L::kVLoads; ++i) dma_v(r, i);
+    for (int i = 0; i < L::kVLoads; ++i) dma_v(t % kNStage, i);
   };
 
   // With few tiles per block the q rows are a large part of what a workgroup
@@ -850,6 +881,11 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
   }
   float hsum = softmax_half(sA, 0);
 
+  // The iteration that computes the scores of a partial tile, the last one if
+  // it reaches past kv_end.
+  const int mask_k0 = kStream ? tile_of(ntiles - 1) * kBKV : 0;
+  const int mask_jt = kStream && mask_k0 + kBKV > kv_end ? ntiles - 2 : -1;
+
   // Iteration jt: S(jt) is in sc with the probabilities of its pairs 0..7
   // already in pw and their per-lane sum in hsum.
   //   phase A: QK of tile jt+1 into sn  ||  pairs 8..15 of tile jt
@@ -858,10 +894,10 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
   // of the loop's four bodies.
   auto iteration = [&](auto stage, int jt, f32x16 (&sc)[2], f32x16 (&sn)[2]) {
     constexpr int S = decltype(stage)::value;
-    const bool has_next = jt + 1 < ntiles;
     // table reads first: their wait joins the tile wait below
-    const int k_next = has_next ? tile_of(jt + 1) * kBKV : 0;
-    const int t_issue = jt + kDist < ntiles ? tile_of(jt + kDist) : 0;
+    const bool has_next = jt + 1 < ntiles;
+    const int k_next = !kStream && has_next ? tile_of(jt + 1) * kBKV : 0;
+    const int t_issue = !kStream && jt + kDist < ntiles ? tile_of(jt + kDist) : 0;
     // tile jt+1 resident (of 4 wavefronts: K of tile jt+1 and V of tile jt)
     // and every wave done with iteration jt-1: the loads of the iteration
     // before were issued that long ago, nothing younger is in flight
@@ -876,14 +912,23 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
     // the interleaved phase; the epilogue drains it).  Of 4 wavefronts, K of
     // tile jt+2 goes into the stage of K(jt), whose scores are done, and V
     // of tile jt+1 into the stage of V(jt-1).
-    TileReqs req = tile_reqs(jt + kDist < ntiles, jt + kDist, t_issue);
-    if constexpr (R != 8)  // (k_next: tile jt+1)
-      req.v = tile_reqs(has_next, jt + 1, k_next / kBKV).v;
+    // DMAs: the K parts first (K is read one phase earlier than V: 0.25-0.45 %
+    // at V7 against interleaving the two)
+    next_k(jt + kDist < ntiles, t_issue);
+    if constexpr (R == 8)
+      next_v(jt + kDist < ntiles, t_issue);
+    else  // (k_next: tile jt+1)
+      next_v(has_next, k_next / kBKV);
     constexpr int NM = QK8 ? 4 : 2 * L::kSteps, NP = L::kLoadsPerTile;
     auto dma = [&](int i) {
 #pragma unroll
       for (int part = 0; part < NP; ++part)
-        if (i == (2 * part + 1) * NM / (2 * NP)) dma_part(req, part);
+        if (i == (2 * part + 1) * NM / (2 * NP)) {
+          if (part < L::kKLoads)
+            dma_k((S + kDist) % kNStage, part);
+          else
+            dma_v((S + (R == 8 ? kDist : 1)) % kNStage, part - L::kKLoads);
+        }
     };
     // second half of tile jt (first half already in pw, its sum in hsum)
     // (On the last tile the QK product runs on a stale or zero-filled LDS
@@ -895,7 +940,15 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
     if (first || wave_any(!(sum <= trip)))
       sum = softmax_fixup(sc, sn, first, m, l, negm, pw, o, shift);
     l += sum;
-    if (has_next && k_next + kBKV > kv_end) mask_tile(sn, k_next, hf, kv_end);
+    if constexpr (!kStream) {
+      if (has_next && k_next + kBKV > kv_end) mask_tile(sn, k_next, hf, kv_end);
+    } else if (jt == mask_jt) {
+      // (laundered: the compiler otherwise works the 32 masks out before the
+      // loop and holds them through it)
+      int k0 = mask_k0;
+      asm volatile("" : "+s"(k0));
+      mask_tile(sn, k0, hf, kv_end);
+    }
     // + pairs 0..7 of tile jt+1.  On the last tile this exponentiates the
     // stale contents of sn into pw words that nothing reads afterwards: one
     // phase-B body in the loop keeps its register allocation within the
