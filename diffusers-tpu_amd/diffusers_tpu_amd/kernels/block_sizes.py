@@ -207,9 +207,10 @@ def launch_plan(batch: int, heads: int, seq_len: int,
   """The launch plan of one attention call on the current GPU.
 
   ``workspace_bytes``: the workspace the call would pass (None: as much as
-  the best plan uses, which is what ``attention`` allocates).  Head dims
-  other than 64 and 128 (and every head dim with ``qk_fp8``) run
-  zero-padded to the kernel's, so they plan as that dim.
+  the best plan uses, which is what ``attention`` allocates at head dims 64
+  and 128).  Other head dims plan here as the next of 64, 128 and 256 (with
+  ``qk_fp8`` they run so, zero-padded).  ``attention`` itself runs the others
+  at their own width, and splits above 128 too, where this plan has no split.
   """
   from diffusers_tpu_amd import _lib
   from diffusers_tpu_amd.kernels.splash import kernel_head_dim

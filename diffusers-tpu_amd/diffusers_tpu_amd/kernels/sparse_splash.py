@@ -3,7 +3,8 @@
 Same arithmetic as ``splash.attention``; the key sweep of each query block
 walks a table of key blocks instead of every block, so skipped blocks cost
 neither memory traffic nor MFMA work (kernels/sparse_splash.py:1-5).  A
-full table reproduces the dense kernel exactly.
+full table reproduces the dense kernel: exactly where that
+sweeps a block's keys in one go, else to bf16 rounding of the probabilities.
 
 The reference's tables are in its own ``(block_q, block_kv)`` units: per
 query block, the sorted key blocks it visits, shared by all heads, or

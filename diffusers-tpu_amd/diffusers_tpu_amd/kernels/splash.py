@@ -26,12 +26,12 @@ Differences a caller can observe, all within the reference's tolerance:
 * As in the reference (kernels/splash.py:607-609,633), ``q * scale *
   log2(e)`` is rounded to bf16 before the QK product (the kernel does this in
   registers with one rounding).
-* Head dims: the kernels are built for 64, 128 and 256.  Any other multiple
-  of 8 runs as it is in the next wider one (``dt_flash_fwd_anydim``); with
-  ``qk_fp8`` dims below 128 run zero-padded (zero channels change no score;
-  the extra output channels are dropped), with the scale of the real dim.  Above 256 (above 128 with ``qk_fp8``) raises
-  ``NotImplementedError``, as does a dim that is not a multiple of 8
-  (kernels/splash.py:156-160).
+* Head dims: any multiple of 8 up to 256 runs as it lies in memory (other
+  than 64 and 128 through ``dt_flash_fwd_anydim``); with ``qk_fp8`` dims
+  below 128 run zero-padded (zero channels change no score; the extra output
+  channels are dropped), with the scale of the real dim.  Above 256 (above
+  128 with ``qk_fp8``) raises ``NotImplementedError``, as does a dim that is
+  not a multiple of 8 (kernels/splash.py:156-160).
 * ``qk_fp8`` casts K to E4M3 in one GPU pass (``fp8_cast``) and the kernel
   casts the scaled q to E4M3 in registers (kernels/splash.py:420-424); the
   QK product runs on the E4M3 MFMA, P and V stay bf16.
@@ -94,8 +94,9 @@ class BlockSizes:
 
 def kernel_head_dim(d, qk_fp8=False):
   """Head dim the gfx950 kernels run for a head dim ``d`` (a multiple of 8):
-  64, 128 or 256; smaller dims are zero-padded up to it (zero channels add
-  nothing to q.k and produce output channels that are dropped).  ``None``
+  64, 128 or 256, the next at or above ``d`` (E4M3 keys and tile tables run
+  zero-padded to it: zero channels add nothing to q.k and produce output
+  channels that are dropped; other calls run at their own width).  ``None``
   above 256, and above 128 with E4M3 keys."""
   if d > 256 or (qk_fp8 and d > 128):
     return None
