@@ -27,12 +27,29 @@ SplitPlan split_plan(int64_t n_wg, int ntiles, int n_cu, int D, int bq,
   constexpr size_t kMaxWs = size_t(512) << 20;
   if (max_ws > kMaxWs) max_ws = kMaxWs;
   const size_t unit_bytes = (size_t)bq * (D + 2) * sizeof(float);
-  int64_t best_ns = 1, best_cost = ntiles + kStartTiles;
+  // Above head dim 128 (bq 128) a tile is 32 keys and short, so a split costs
+  // more of them: 6 tiles for the merge's launch, 11 for writing and reading
+  // 256 parts' outputs, and 15 % a tile when all CUs are busy instead of few.
+  // Measured, whole against split (us): D = 256, 128 blocks of 14 tiles 24.6,
+  // 32.5 in 2, of 32 tiles 38.7, 42.2, of 64 tiles 63.7, 61.2; 64 blocks of 14
+  // tiles 24.1, 25.7, of 32 tiles 37.8, 31.3 in 3; D = 160, 128 blocks of 14
+  // tiles 19.1, 25.3, of 64 tiles 53.3, 43.3.
+  const bool wide = bq == 128;
+  auto cost_of = [&](int64_t ns) -> double {
+    const int64_t units = rem * ns, rounds = (units + n_cu - 1) / n_cu;
+    const double tiles = (double)((ntiles + ns - 1) / ns);
+    if (!wide)
+      return (double)rounds * (tiles + kStartTiles) +
+             (double)(ns > 1 ? ns * kMergeTiles : 0);
+    const double busy = units < n_cu ? (double)units / n_cu : 1.0;
+    return (double)rounds * (tiles * (1 + 0.15 * busy) + 2 * kStartTiles) +
+           (ns > 1 ? 6 + 11 * (double)units / n_cu : 0.0);
+  };
+  int64_t best_ns = 1;
+  double best_cost = cost_of(1);
   for (int64_t ns = 2; ns <= kMaxSplit && ns <= ntiles / 2; ++ns) {
     if ((size_t)(rem * ns) * unit_bytes > max_ws) break;
-    const int64_t rounds = (rem * ns + n_cu - 1) / n_cu;
-    const int64_t cost =
-        rounds * ((ntiles + ns - 1) / ns + kStartTiles) + ns * kMergeTiles;
+    const double cost = cost_of(ns);
     if (cost < best_cost) {
       best_cost = cost;
       best_ns = ns;

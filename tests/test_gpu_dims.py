@@ -100,3 +100,12 @@ def test_fixed_m_and_device_lengths(sp, d):
   assert not got[1].any()
   o, m, l = sp.residual_attention(q, k, v, kv_len=n)
   assert not o[1].any() and not m[1].any() and not l[1].any()
+
+
+@pytest.mark.parametrize("d", [136, 256])
+def test_wide_dims_split_only_long_sweeps(sp, d):
+  """Half a round of workgroups is split over 4096 keys and not over 424,
+  where the merge would cost more than the idle CUs."""
+  banner(f"wide split plan d={d}")
+  assert sp._split_bytes(2, 16, 424, 424, 424, d, 0) == 0
+  assert sp._split_bytes(2, 16, 424, 4096, 4096, d, 0) > 0
