@@ -206,7 +206,9 @@ __device__ __forceinline__ float softmax_fixup(f32x16 (&s)[2], f32x16 (&sn)[2],
   mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
   // (scores are relative to m - shift: the row's max is mx - shift above m)
   const float delta = first ? mx - shift : fmaxf(mx - shift, 0.f);
-  const float alpha = __builtin_amdgcn_exp2f(-delta);
+  // (nothing to rescale on the first tile, whose max may lie any distance
+  // below 0: exp2(-delta) would overflow and turn the zero sums into NaN)
+  const float alpha = first ? 1.0f : __builtin_amdgcn_exp2f(-delta);
   m += delta;
 #pragma unroll
   for (int r = 0; r < 16; ++r) negm[r] = -m;

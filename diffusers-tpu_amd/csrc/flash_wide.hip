@@ -408,7 +408,9 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
       for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sc[r]);
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
       const float delta = first ? mx - shift : fmaxf(mx - shift, 0.f);
-      const float alpha = __builtin_amdgcn_exp2f(-delta);
+      // (the first tile has nothing to rescale: its max may lie so far below
+      // 0 that exp2(-delta) overflows, and 0 * inf is NaN)
+      const float alpha = first ? 1.0f : __builtin_amdgcn_exp2f(-delta);
       m += delta;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
