@@ -151,6 +151,11 @@ constexpr float kTripShifted = kTripSum * 16777216.0f;  // 2^(12 + 24)
 template <int N>
 using IC = std::integral_constant<int, N>;  // a compile-time ring stage
 constexpr float kFixedRecenter = 88.0f;  // kernels/fixed_m_bound.py:42
+// A first reference this far (log2 units) below another key group's is a
+// masked tile's: taken as it is, the first real score would be re-based from
+// it with the rounding of that distance (2^-13 here, everything at a mask of
+// the type's lowest value; -inf gives NaN).
+constexpr float kRefGap = 2048.0f;
 
 // scores of keys at or past kv_end -> -inf.  Bit arithmetic (a sign mask
 // and a bitfield select) rather than 32 compares, which would each claim a
@@ -192,18 +197,22 @@ __device__ __forceinline__ float dot2_sum(uint32_t w, float acc) {
 // Rare path: raise the reference m of the lane's row to the row max of the
 // tile in s (on the first tile: set it to that max), re-base the scores of s
 // and of the already computed next tile sn, recompute the probabilities of s
-// and rescale l and O.  Scores are relative to the old m on entry.
+// and rescale l and O.  Scores are relative to the old m on entry.  `other`
+// (first tile only): the largest row max of the key groups' first tiles, or
+// -inf; it takes the place of a max more than kRefGap below it.
 template <int NB>
 __device__ __forceinline__ float softmax_fixup(f32x16 (&s)[2], f32x16 (&sn)[2],
                                                bool first, float& m, float& l,
                                                f32x16& negm, uint32_t (&pw)[16],
-                                               f32x16 (&o)[NB], float shift) {
+                                               f32x16 (&o)[NB], float shift,
+                                               float other) {
   float mx = s[0][0];
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[kb][r]);
   mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  if (first && mx < other - kRefGap) mx = other;
   // (scores are relative to m - shift: the row's max is mx - shift above m)
   const float delta = first ? mx - shift : fmaxf(mx - shift, 0.f);
   // (nothing to rescale on the first tile, whose max may lie any distance
@@ -883,6 +892,21 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
   }
   float hsum = softmax_half(sA, 0);
 
+  // Key groups: each leaves its row maxes of its first tile behind the rings
+  // (read in iteration 0, past its barrier): a group that starts on masked
+  // keys takes another's for its reference, as one sweep has tile 0's.
+  typedef __attribute__((address_space(3))) float lds_f32;
+  lds_f32* first_max = (lds_f32*)(lds + G * L::kLds) + wave * 32 + l32;
+  if constexpr (G > 1) {
+    float mx = sA[0][0];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sA[kb][r]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (hf == 0) first_max[grp * BQ] = ntiles > 0 ? mx : -INFINITY;
+  }
+
   // The iteration that computes the scores of a partial tile, the last one if
   // it reaches past kv_end.
   const int mask_k0 = kStream ? tile_of(ntiles - 1) * kBKV : 0;
@@ -939,8 +963,15 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
     // the branch, out of the MFMA interleave.)
     float sum = hsum + phase_a(T{}, IC<(S + 1) % kNStage>{}, sn, sc, dma);
     const bool first = jt == 0 && !fixed;
-    if (first || wave_any(!(sum <= trip)))
-      sum = softmax_fixup(sc, sn, first, m, l, negm, pw, o, shift);
+    if (first || wave_any(!(sum <= trip))) {
+      float other = -INFINITY;
+      if constexpr (G > 1)
+        if (first) {
+#pragma unroll
+          for (int g = 0; g < G; ++g) other = fmaxf(other, first_max[g * BQ]);
+        }
+      sum = softmax_fixup(sc, sn, first, m, l, negm, pw, o, shift, other);
+    }
     l += sum;
     if constexpr (!kStream) {
       if (has_next && k_next + kBKV > kv_end) mask_tile(sn, k_next, hf, kv_end);
@@ -991,7 +1022,6 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
     constexpr int kPart = D * 32 * 4 + 512;  // bytes of a wavefront's o, m, l
     static_assert((G - 1) * R * kPart <= G * L::kLds, "parts fit the rings");
     typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
-    typedef __attribute__((address_space(3))) float lds_f32;
     if (grp > 0) {
       lds_u8* part_o = lds + ((grp - 1) * R + wave) * kPart;
 #pragma unroll
@@ -1140,8 +1170,10 @@ int launch_flash(const FlashParams& base, hipStream_t st) {
   constexpr int D = HD::D;
   using L = Stage<HD, QK8, R>;
   constexpr int BQ = R * 32;
-  // (4 x 1: room for the q rows of two wavefronts behind the ring)
-  constexpr int kLdsBytes = G * L::kLds + (R == 4 && G == 1 ? 2 * 32 * 2 * D : 0);
+  // (4 x 1: room for the q rows of two wavefronts behind the ring; key groups:
+  // a row max each)
+  constexpr int kLdsBytes = G * L::kLds + (R == 4 && G == 1 ? 2 * 32 * 2 * D : 0) +
+                            (G > 1 ? G * BQ * 4 : 0);
   FlashParams p = base;
   p.n_qblk = (p.Sq + BQ - 1) / BQ;
   const int64_t nwg = (int64_t)p.n_qblk * p.Hq * p.B;

@@ -66,6 +66,7 @@ constexpr float kWTrip = 4096.0f;
 constexpr float kWShift = 24.0f;          // online heads' reference offset
 constexpr float kWTripShifted = kWTrip * 16777216.0f;  // 2^(12 + 24)
 constexpr float kWRecenter = 88.0f;       // kernels/fixed_m_bound.py:42
+constexpr float kWRefGap = 2048.0f;       // see `low` in the prologue
 
 template <int N>
 using WStage = std::integral_constant<int, N>;
@@ -183,9 +184,11 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
   int kv_end =
       resolve_len(p.kv_len_dev, p.kv_len_count, b, p.kv_end, p.Skv);
   int ntiles = (kv_end + kWBKV - 1) / kWBKV;
+  const uint16_t* kfirst = kbase;  // tile 0 of the whole sweep
+  int tbeg = 0;
   if (unit >= 0) {
     // a split part's share of the tiles, as keys and values of its own
-    const int tbeg = (ntiles * part) / p.n_split;
+    tbeg = (ntiles * part) / p.n_split;
     ntiles = (ntiles * (part + 1)) / p.n_split - tbeg;
     kbase += (int64_t)tbeg * kWBKV * p.k_ss;
     vbase += (int64_t)tbeg * kWBKV * p.v_ss;
@@ -399,14 +402,16 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
   // leaves its range), recompute their probabilities into pw, shift the
   // already computed next tile's scores sn and rescale l and O.  Then add
   // the tile's sum to l.
+  // `low` (first tile only): the row max of the whole sweep's tile 0, or -inf.
   auto settle = [&](bool first, const f32x16& sc, uint32_t (&pw)[8],
-                    float sum, f32x16& sn) {
+                    float sum, f32x16& sn, float low) {
     if (first || wave_any(!(sum <= trip))) {
       mfma_drain();  // sn is written by the QK assembly
       float mx = sc[0];
 #pragma unroll
       for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sc[r]);
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      if (first && mx < low - kWRefGap) mx = low;
       const float delta = first ? mx - shift : fmaxf(mx - shift, 0.f);
       // (the first tile has nothing to rescale: its max may lie so far below
       // 0 that exp2(-delta) overflows, and 0 * inf is NaN)
@@ -439,14 +444,42 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
   // ---- prologue: K of tiles 0 and 1, then what iterations -3 and -2
   // would request; S(0) and S(1); after every wave is done with K stage 0,
   // iteration -1's request (K(4) goes there); P(0) with the first re-base.
+  //
+  // A split part other than the first also scores tile 0 of the whole sweep
+  // (through V stage 3, which nothing fills before iteration 0): `low`, its
+  // row max, stands in for the max of a first tile more than 2048 below it.
+  // Such a tile holds masked keys, and a reference taken from it would turn
+  // the part's later, real scores into NaN (-inf) or round them away (the
+  // type's lowest value), where one sweep from tile 0 gets them right.
+  if (tbeg > 0) {
+    const u32x4 rsrc = make_rsrc((uint64_t)(uintptr_t)kfirst, kWBKV * krow);
+#pragma unroll
+    for (int i = 0; i < kWLoads; ++i)
+      lds_dma16_buf(rsrc, kvo[i], lds_v + 3 * kWTileB + i * 1024);
+  }
   issue_k(0);
   issue_k(1);
   issue_k(2);
   issue_v(0);
   issue_k(3);
   issue_v(1);
-  wait_vmcnt_c<2 * kWGroup>();  // K(0) and K(1) landed
+  wait_vmcnt_c<2 * kWGroup>();  // K(0) and K(1) landed (and tile 0 above)
   __syncthreads();
+  float low = -INFINITY;
+  if (tbeg > 0) {
+    auto kfld = [&](int t) {
+      return __builtin_bit_cast(
+          bf16x8, *(const __attribute__((address_space(3))) u32x4*)(
+                      lds + kread[t & 7] + (kWVOff + 3 * kWTileB + 256 * (t >> 3))));
+    };
+    f32x16 s0 = qk_first(kfld(0), qf[0], negm);
+#pragma unroll
+    for (int t = 1; t < kWSteps; ++t) qk_acc(s0, kfld(t), qf[t]);
+    mfma_drain();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) low = fmaxf(low, s0[r]);
+    low = fmaxf(low, __shfl_xor(low, 32, 64));
+  }
   f32x16 sA, sB;
   sB = qk_first(kld(WStage<0>{}, 0), qf[0], negm);
   sA = qk_first(kld(WStage<1>{}, 0), qf[0], negm);
@@ -473,7 +506,7 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
       else
         sa = dot2_acc(pwA[i], sa);
     }
-    settle(!fixed, sB, pwA, sa + sb, sA);
+    settle(!fixed, sB, pwA, sa + sb, sA, low);
   }
 
   // Iteration j (ring stage S = j % 4 of V, (j + 2) % 4 of K): on entry sc
@@ -579,7 +612,7 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
       valu_beside(2 * i + 1);
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (j + 1 < ntiles) settle(false, sc, pwn, sa + sb, sn);
+    if (j + 1 < ntiles) settle(false, sc, pwn, sa + sb, sn, -INFINITY);
     if (j + 2 < ntiles && (j + 3) * kWBKV > kv_end) {
       mfma_drain();
       wide_mask(sn, (j + 2) * kWBKV, hf, kv_end);

@@ -1,5 +1,8 @@
-"""Rows whose scores lie far from zero.  The kernels keep one reference per
-row, set on the first tile they sweep."""
+"""Rows whose scores lie far from zero, and keys that only some tiles see:
+the kernels keep one reference per row, taken from the first tile they sweep,
+so scores far below zero there, or a tile of masked keys (a channel that gives
+-inf, or the type's lowest value) at the start of a key group's or a split
+part's share must not reach the result."""
 import numpy as np
 import pytest
 import torch
@@ -47,3 +50,26 @@ def test_scores_far_below_zero(dta, d, shape):
   o, m, l = dta.residual_attention(q, k, v)
   assert_attn_close(to64((o / l)[:, h][:, :, rows]), want, "residual")
 
+
+# (B, H, Sq, Skv, D): 4 x 2 and 2 x 4 key groups; split parts above head dim
+# 128 (one sweep each before they were split)
+MASKED = [(2, 22, 250, 1500, 128), (1, 8, 1000, 1024, 64), (1, 24, 300, 1500, 72),
+          (1, 2, 300, 4096, 256), (1, 3, 200, 2500, 136)]
+
+
+@pytest.mark.parametrize("low", [float("-inf"), torch.finfo(torch.bfloat16).min])
+@pytest.mark.parametrize("case", MASKED, ids=[str(c) for c in MASKED])
+def test_masked_tiles_after_the_first(dta, case, low):
+  """All keys but tile 0 and a few of the last ones masked by a channel."""
+  b, h, sq, skv, d = case
+  banner(f"masked tiles {case} {low}")
+  q, k, v = _inputs(b, h, sq, skv, d, 660)
+  q[..., 0], k[..., 0] = 1.0, 0.0
+  keep = np.r_[0:64, skv - 5:skv]
+  want = A.attention_f64(to64(q[:1, :2]), to64(k[:1, :2, keep]),
+                         to64(v[:1, :2, keep]))
+  k[:, :, 64:skv - 5, 0] = low
+  got = dta.attention(q, k, v)
+  assert_attn_close(to64(got[:1, :2]), want, "masked")
+  o, m, l = dta.residual_attention(q, k, v)
+  assert_attn_close(to64((o / l)[:1, :2]), want, "residual")
