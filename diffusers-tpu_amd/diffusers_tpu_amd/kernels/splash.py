@@ -372,6 +372,27 @@ def _plain_rows(t):
   return t
 
 
+def _memory_overlaps(a, b):
+  """Whether the storages of two tensors share memory (also as storages of
+  their own over one allocation, as DLPack makes them)."""
+  sa, sb = a.untyped_storage(), b.untyped_storage()
+  pa, pb = sa.data_ptr(), sb.data_ptr()
+  return pa < pb + sb.nbytes() and pb < pa + sa.nbytes()
+
+
+def _writes_like_copy(out, *reads):
+  """Whether a kernel that writes ``out`` while it reads ``reads`` does what
+  ``out.copy_(result)`` does: the rows where the kernel's stores can put them,
+  one element a position, memory that nothing read shares, and no autograd
+  rule that ``copy_`` would apply or enforce."""
+  return (type(out) is torch.Tensor and out.data_ptr() % 8 == 0 and
+          not any(st == 0 and n > 1
+                  for n, st in zip(out.shape, out.stride())) and
+          not (out.requires_grad and torch.is_grad_enabled()) and
+          (not out.is_inference() or torch.is_inference_mode_enabled()) and
+          not any(_memory_overlaps(out, t) for t in reads if t is not None))
+
+
 def _call_anydim(query, key, value, scale, n, out, residual, mk, workspace):
   """One ``dt_flash_fwd_anydim`` call (arguments checked by ``_launch``;
   ``n`` as in ``_call_ex``)."""
@@ -392,10 +413,9 @@ def _call_anydim(query, key, value, scale, n, out, residual, mk, workspace):
       l = torch.empty((b, hq, sq, 1), device=dev, dtype=torch.float32)
       outs = (None, None, o.data_ptr(), m.data_ptr(), l.data_ptr())
     else:
-      # an output that shares memory with an input is written after the call
-      direct = out is not None and all(
-          out.untyped_storage().data_ptr() != t.untyped_storage().data_ptr()
-          for t in (q, k, v))
+      # an output that the kernel cannot write in place of a copy is written
+      # after the call
+      direct = out is not None and _writes_like_copy(out, q, k, v, mk, n_dev)
       o = out if direct else torch.empty((b, hq, sq, d), device=dev,
                                          dtype=torch.bfloat16)
       outs = (o.data_ptr(), s3(o), None, None, None)
@@ -414,7 +434,13 @@ def _call_anydim(query, key, value, scale, n, out, residual, mk, workspace):
         _lib.raw_stream(dev.index)))
   if residual:
     return o, m, l
-  return o if out is None else out if direct else out.copy_(o)
+  if out is None:
+    return o
+  if not direct:
+    return out.copy_(o)
+  if not out.is_inference():
+    torch.autograd.graph.increment_version(out)  # written in place
+  return out
 
 
 @functools.lru_cache(maxsize=4096)
