@@ -364,11 +364,17 @@ def _launch(query, key, value, scale, kv_len, out=None, residual=False,
 
 def _plain_rows(t):
   """``_as_bf16_rows`` with rows that do not overlap (an expanded or
-  sliding-window view is copied) in a (b, h) slice below 4 GiB - 256."""
+  sliding-window view is copied) in a (b, h) slice below 4 GiB - 256, at an
+  address and strides that the kernels take: ``contiguous()`` keeps those of a
+  tensor it finds contiguous, such as a view that starts 8 bytes into a buffer
+  or an axis of one element with a stride of its own."""
   t = _as_bf16_rows(t)
   s, d = t.shape[2:]
   if (s > 1 and t.stride(2) < d) or s * t.stride(2) * 2 >= (1 << 32) - 256:
     t = t.contiguous()
+  if (t.data_ptr() & 15 or any(st & 7 for st in t.stride()[:3]) or
+      t.stride(2) < d):
+    t = t.clone(memory_format=torch.contiguous_format)
   return t
 
 
