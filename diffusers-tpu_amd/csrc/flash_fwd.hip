@@ -127,6 +127,13 @@ int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
                        "dt_flash_fwd: strides must be multiples of 8 elements "
                        "(16 for E4M3 keys)");
   }
+  // a (b, h) slice is read as rows of its row stride (one key: any stride)
+  const int64_t k_ss = Skv > 1 ? k_strides[2] : D;
+  const int64_t v_ss = packed ? 0 : Skv > 1 ? v_strides[2] : D;
+  if (k_ss < D || (!packed && v_ss < D))
+    return set_error(DT_ERR_UNSUPPORTED,
+                     "dt_flash_fwd: key or value rows overlap (row stride "
+                     "below the head dim %d)", D);
   if (!al16(q) || !al16(k) || (!packed && !al16(v)) || (o && ((uintptr_t)o & 7u)) ||
       (o32 && !al16(o32)))
     return set_error(DT_ERR_UNSUPPORTED, "dt_flash_fwd: misaligned tensor");
@@ -151,10 +158,10 @@ int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
   p.q_ss = q_strides[2];
   p.k_sb = k_strides[0];
   p.k_sh = k_strides[1];
-  p.k_ss = k_strides[2];
+  p.k_ss = k_ss;
   p.v_sb = packed ? 0 : v_strides[0];
   p.v_sh = packed ? 0 : v_strides[1];
-  p.v_ss = packed ? 0 : v_strides[2];
+  p.v_ss = v_ss;
   if (o) {
     p.o_sb = o_strides[0];
     p.o_sh = o_strides[1];

@@ -195,7 +195,7 @@ def _launch_sparse(query, key, value, scale, kv_len, table, *, residual,
     from .fp8_cast import quantize_saturating
     k, k_format = quantize_saturating(key), 1
   else:
-    k, k_format = splash._as_bf16_rows(key), 0
+    k, k_format = splash._key_rows(key), 0
   if mk is not None:
     mk = splash._mk_operand(mk, hq, q.device)
   mk_ptr = None if mk is None else mk.data_ptr()
@@ -207,6 +207,8 @@ def _launch_sparse(query, key, value, scale, kv_len, table, *, residual,
   packed = None
   if n * table.kept_tiles >= splash.PACKED_V_MIN_KEYS * table.full_tiles:
     packed = splash.pack_v(v, n)
+  else:
+    v = splash._key_rows(v)
   return splash._call_ex(q, k, k_format, v, packed, None, residual, hkv, skv,
                          scale, n, mk_ptr, span, ids)
 

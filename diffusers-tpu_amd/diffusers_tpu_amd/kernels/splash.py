@@ -76,6 +76,16 @@ def _as_bf16_rows(t):
   return t
 
 
+def _key_rows(t):
+  """``_as_bf16_rows`` of keys or values, without rows that overlap or repeat
+  (an expanded or sliding-window view is copied): the kernels read a (b, h)
+  slice as rows of its row stride and nothing past the last one."""
+  t = _as_bf16_rows(t)
+  if t.shape[2] > 1 and t.stride(2) < t.shape[3]:
+    t = t.contiguous()
+  return t
+
+
 class BlockSizes:
   """The reference's per-call tiling record (kernels/splash.py:92-112):
   ``block_q``, ``block_kv`` and ``block_kv_compute`` (default ``block_kv``).
@@ -229,7 +239,8 @@ def _launch_plain(query, key, value, scale, kv_len, residual, workspace):
   qp, kp, vp = query.data_ptr(), key.data_ptr(), value.data_ptr()
   if (qst[3] != 1 or kst[3] != 1 or vst[3] != 1 or (qp | kp | vp) & 15 or
       (qst[0] | qst[1] | qst[2] | kst[0] | kst[1] | kst[2] | vst[0] | vst[1] |
-       vst[2]) & 7):
+       vst[2]) & 7 or
+      (skv > 1 and (kst[2] < d or vst[2] < d))):
     return None
   len_ptr = None
   if kv_len is None:
@@ -345,7 +356,7 @@ def _launch(query, key, value, scale, kv_len, out=None, residual=False,
     from .fp8_cast import quantize_saturating
     k = quantize_saturating(key)
   else:
-    k = _as_bf16_rows(key)
+    k = _key_rows(key)
   if mk is not None:
     mk = _mk_operand(mk, hq, q.device)
   mk_ptr = None if mk is None else mk.data_ptr()
@@ -358,19 +369,19 @@ def _launch(query, key, value, scale, kv_len, out=None, residual=False,
           workspace.packed_v(packed_v_numel(b, hkv, skv if n_dev is not None
                                             else n))
       packed_v = pack_v(v, length, out=buf)
+  if packed_v is None:
+    v = _key_rows(v)
   return _call_ex(q, k, 1 if qk_fp8 else 0, v, packed_v, out, residual,
                   hkv, skv, scale, length, mk_ptr, workspace=workspace)
 
 
 def _plain_rows(t):
-  """``_as_bf16_rows`` with rows that do not overlap (an expanded or
-  sliding-window view is copied) in a (b, h) slice below 4 GiB - 256, at an
-  address and strides that the kernels take: ``contiguous()`` keeps those of a
+  """``_key_rows`` in a (b, h) slice below 4 GiB - 256, at an address and strides that the kernels take: ``contiguous()`` keeps those of a
   tensor it finds contiguous, such as a view that starts 8 bytes into a buffer
   or an axis of one element with a stride of its own."""
-  t = _as_bf16_rows(t)
+  t = _key_rows(t)
   s, d = t.shape[2:]
-  if (s > 1 and t.stride(2) < d) or s * t.stride(2) * 2 >= (1 << 32) - 256:
+  if s * t.stride(2) * 2 >= (1 << 32) - 256:
     t = t.contiguous()
   if (t.data_ptr() & 15 or any(st & 7 for st in t.stride()[:3]) or
       t.stride(2) < d):

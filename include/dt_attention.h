@@ -56,6 +56,8 @@
  * Conventions shared by every entry point:
  *   - Tensors are bf16 bit patterns (uint16_t) in device memory; the last
  *     (head-dim) axis is contiguous; other axes are given by element strides.
+ *     The attention entry points refuse key or value rows that overlap (a row
+ *     stride below D with more than one key; DT_ERR_UNSUPPORTED).
  *   - `stream` is a hipStream_t passed as void* (NULL = default stream).
  *   - No entry point allocates, frees or synchronizes; all work is enqueued on
  *     `stream`.  There is no mutable global state apart from the static
@@ -428,9 +430,8 @@ size_t dt_flash_fwd_workspace_bytes(int B, int Hq, int Sq, int Skv,
  * dt_flash_fwd_ex with bf16 keys, row-major V and no tile table, at any head
  * dim that is a multiple of 8 up to 256 (kernels/splash.py:156-160): rows of
  * D elements are read and written as they are, at the arithmetic of the dim
- * itself, with the tail split at every dim.  Rows of one (b, h) slice of q, k, v must not overlap
- * (stride s >= D, or one row), and a K or V slice must span less than 4 GiB -
- * 256.  The default scale is 1/sqrt(D).
+ * itself, with the tail split at every dim.  A K or V slice must span less
+ * than 4 GiB - 256.  The default scale is 1/sqrt(D).
  */
 int dt_flash_fwd_anydim(const uint16_t* q, const uint16_t* k,
                         const uint16_t* v, uint16_t* o, int B, int Hq, int Hkv,

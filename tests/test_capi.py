@@ -225,3 +225,28 @@ def test_binding_matches_the_header_prototypes():
     ret, params = protos[name]
     assert _ctype_of(ret) == res, (name, ret)
     assert [_ctype_of(p) for p in params] == list(args), name
+
+
+def test_overlapping_key_rows_are_refused():
+  """A (b, h) slice of K or V is read as rows of its row stride: a stride
+  below the head dim (0: an expanded row) would be read as zeros."""
+  lib = _lib.load()
+  fake = ctypes.c_void_p(0x1000)
+  for d in (64, 128, 256):
+    good = _lib.i64_array(64 * d, 64 * d, d)
+    for stride in (0, 8, d - 8):
+      bad = _lib.i64_array(64 * d, 64 * d, stride)
+      for ks, vs in ((bad, good), (good, bad)):
+        calls = [
+            lib.dt_flash_fwd(fake, fake, fake, fake, 1, 1, 1, 8, 8, d, good,
+                             ks, vs, good, 0.0, 0, None, None, None, None,
+                             None),
+            lib.dt_flash_fwd_ex(fake, fake, 0, fake, vs, None, 0, fake, 1, 1,
+                                1, 8, 8, d, good, ks, good, 0.0, 0, None, None,
+                                None, None, None, None, None, None, 0, None),
+            lib.dt_flash_fwd_anydim(fake, fake, fake, fake, 1, 1, 1, 8, 8, d,
+                                    good, ks, vs, good, 0.0, 0, None, None,
+                                    None, None, None, None, 0, None)]
+        for rc in calls:
+          assert rc == _lib.DT_ERR_UNSUPPORTED
+          assert b"overlap" in lib.dt_last_error()
