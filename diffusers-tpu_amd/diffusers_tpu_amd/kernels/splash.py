@@ -671,14 +671,15 @@ def _merge_kernel_ok(parts):
   """Whether ``merge_residuals`` may call ``dt_merge_residuals`` on these
   triples: plain contiguous float32 GPU tensors, and nothing that records,
   transforms or traces torch operations (autograd, ``torch.func``, dispatch
-  and function modes, ``torch.compile``)."""
+  and function modes, ``torch.compile``, ``torch.jit.trace``, ``torch.fx``
+  proxies)."""
   if not 1 <= len(parts) <= _lib.MERGE_MAX_PARTS or any(
-      len(p) != 3 for p in parts):
+      not isinstance(p, (tuple, list)) or len(p) != 3 for p in parts):
     return False
   ts = [t for p in parts for t in p]
   if not all(type(t) is torch.Tensor for t in ts):
     return False
-  if (torch.compiler.is_compiling() or
+  if (torch.compiler.is_compiling() or torch.jit.is_tracing() or
       torch.overrides._get_current_function_mode_stack() or
       torch.utils._python_dispatch._get_current_dispatch_mode() is not None or
       torch._C._functorch.peek_interpreter_stack() is not None or

@@ -81,3 +81,22 @@ def test_merge_other_calls_go_through_torch(sp):
   far = [(p[0], torch.full_like(p[1], v), p[2])
          for p, v in zip(parts, (-300.0, 100.0))]
   assert torch.equal(sp.merge_residuals(far), parts[1][0] / parts[1][2])
+
+
+def test_merge_under_tracers(sp):
+  """torch.jit.trace records the operations, and torch.fx passes proxies."""
+  banner("merge: tracers")
+  parts = _parts(2, (1, 2, 9, 8))
+  other = _parts(2, (1, 2, 9, 8), seed=611)
+  flat = lambda ps: tuple(t for p in ps for t in p)
+  f = lambda *ts: sp.merge_residuals([ts[:3], ts[3:]])
+  traced = torch.jit.trace(f, flat(parts))
+  assert torch.allclose(traced(*flat(other)), _merge64(other).float(),
+                        rtol=1e-4, atol=1e-4)
+
+  def g(a, b):  # a, b: a part each, as one tensor of three planes
+    return sp.merge_residuals([a, b])
+  graph = torch.fx.symbolic_trace(g)
+  ab = [torch.stack(torch.broadcast_tensors(*p)) for p in other]
+  assert torch.allclose(graph(*ab), _merge64(other).float(), rtol=1e-4,
+                        atol=1e-4)
