@@ -3,8 +3,11 @@
 Same arithmetic as ``splash.attention``; the key sweep of each query block
 walks a table of key blocks instead of every block, so skipped blocks cost
 neither memory traffic nor MFMA work (kernels/sparse_splash.py:1-5).  A
-full table reproduces the dense kernel: exactly where that
-sweeps a block's keys in one go, else to bf16 rounding of the probabilities.
+full table (``kv_table`` lists, or ``None``) reproduces the dense call exactly:
+it runs as ``splash`` runs the call without one.  A ``TileTable`` is swept as
+its tensors say when the kernel runs, always in 256-row workgroups; where the
+dense call runs in other shapes, a full one agrees with it to bf16 rounding of
+the probabilities.
 
 The reference's tables are in its own ``(block_q, block_kv)`` units: per
 query block, the sorted key blocks it visits, shared by all heads, or
@@ -162,7 +165,8 @@ def _dyn_table(kv_table_dyn):
 
 
 def _launch_sparse(query, key, value, scale, kv_len, table, *, residual,
-                   mk=None, qk_fp8=False):
+                   mk=None, qk_fp8=False, dense=False):
+  """``dense``: the table visits every key below ``kv_len``."""
   for nm, t in (("query", query), ("key", key), ("value", value)):
     splash._check_bhsd(nm, t)
   splash._check_same_device(query.device, key=key, value=value)
@@ -173,6 +177,14 @@ def _launch_sparse(query, key, value, scale, kv_len, table, *, residual,
   if d % 8 or d > 128:
     raise NotImplementedError(f"head_dim={d}: block-sparse attention covers "
                               "multiples of 8 up to 128")
+  if hq % hkv:
+    raise ValueError(f"{hq} query heads not a multiple of {hkv} kv heads")
+  n = _host_kv_len(kv_len, skv)
+  if table.sq != sq or table.kv_len != n or table.span.shape[0] != hq:
+    raise ValueError("TileTable was built for another shape or kv_len")
+  if dense and (scale is None or scale > 0):
+    return splash._launch(query, key, value, scale, n, residual=residual,
+                          mk=mk, qk_fp8=qk_fp8)
   if d != 128:
     # zero-padded channels: same scores; the extra output channels dropped
     scale = 1.0 / math.sqrt(d) if scale is None else float(scale)
@@ -183,11 +195,6 @@ def _launch_sparse(query, key, value, scale, kv_len, table, *, residual,
     if residual:
       return res[0][..., :d].contiguous(), res[1], res[2]
     return res[..., :d].contiguous()
-  if hq % hkv:
-    raise ValueError(f"{hq} query heads not a multiple of {hkv} kv heads")
-  n = _host_kv_len(kv_len, skv)
-  if table.sq != sq or table.kv_len != n or table.span.shape[0] != hq:
-    raise ValueError("TileTable was built for another shape or kv_len")
   scale = 1.0 / math.sqrt(d) if scale is None else float(scale)
   q = splash._as_bf16_rows(query)
   v = splash._as_bf16_rows(value)
@@ -237,6 +244,12 @@ def _table_for(query, key, block_q, block_kv, kv_table, kv_table_dyn, kv_len):
                           block_kv=block_kv, kv_len=n, device=query.device)
 
 
+def _visits_all(table, kv_table):
+  """Whether a table made in this call keeps every tile (a caller's own
+  ``TileTable`` may have been written to since it was built)."""
+  return table is not kv_table and table.kept_tiles == table.full_tiles
+
+
 def attention(query, key, value, *, scale=None, block_q, block_kv,
               block_kv_compute=None, use_fixed_m=False, qk_fp8=False,
               kv_table=None, kv_table_dyn=None, kv_len=None):
@@ -251,9 +264,10 @@ def attention(query, key, value, *, scale=None, block_q, block_kv,
   del block_kv_compute
   table = _table_for(query, key, block_q, block_kv, kv_table, kv_table_dyn,
                      kv_len)
+  dense = _visits_all(table, kv_table)
   mk = splash._fixed_m_operand(query, key, scale) if use_fixed_m else None
   out = _launch_sparse(query, key, value, scale, kv_len, table,
-                       residual=False, mk=mk, qk_fp8=qk_fp8)
+                       residual=False, mk=mk, qk_fp8=qk_fp8, dense=dense)
   return out if query.dtype == torch.bfloat16 else out.to(query.dtype)
 
 
@@ -274,4 +288,4 @@ def residual_attention(query, key, value, *, scale=None, block_q, block_kv,
                      kv_len)
   return _launch_sparse(query, key, value, scale, kv_len, table,
                         residual=True, mk=mk if use_fixed_m else None,
-                        qk_fp8=qk_fp8)
+                        qk_fp8=qk_fp8, dense=_visits_all(table, kv_table))

@@ -161,3 +161,26 @@ def test_sparse_head_dim_96(sp):
   mask = SP.block_mask(seq, seq, 256, 256, table)
   want = SP.attention_masked_f64(to64(q), to64(k), to64(v), mask)
   assert_attn_close(to64(got), want, "sparse d=96")
+
+
+@pytest.mark.parametrize("d", [64, 72, 128])
+@pytest.mark.parametrize("shape", [(1, 8, 1000, 1024), (2, 4, 700, 900),
+                                   (1, 3, 300, 4096)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_full_table_through_the_entry_points(sp, d, shape, residual):
+  """``attention`` and ``residual_attention`` with every key block listed give
+  the dense call's bits, in whatever workgroup shape or split that runs."""
+  import diffusers_tpu_amd as dta
+  banner(f"full table d={d} {shape}")
+  b, h, sq, skv = shape
+  q = seeded((b, h, sq, d), 123)
+  k = seeded((b, h, skv, d), 124)
+  v = seeded((b, h, skv, d), 125)
+  name = "residual_attention" if residual else "attention"
+  for n in (None, skv - 70):
+    for fp8 in (False, True):
+      got = getattr(sp, name)(q, k, v, block_q=512, block_kv=512, kv_len=n,
+                              qk_fp8=fp8)
+      want = getattr(dta, name)(q, k, v, kv_len=n, qk_fp8=fp8)
+      for x, y in zip(got, want) if residual else ((got, want),):
+        assert torch.equal(x, y), (n, fp8)
