@@ -31,6 +31,7 @@ void clear_error() { g_msg[0] = 0; }
 //   no keys / rows (the empty result) instead of all of them.  Callers
 //   gate on dt_version() >= 300.
 // 0.3.1: dt_merge_residuals, dt_flash_fwd_anydim.
-extern "C" int dt_version(void) { return 301; }
+// 0.3.2: dt_flash_fwd_shape.
+extern "C" int dt_version(void) { return 302; }
 
 extern "C" const char* dt_last_error(void) { return dt::g_msg; }

@@ -103,21 +103,25 @@ int device_cu_count(int* n_cu) {
 // 33.6 -> 29.6, H96 S1024 70.1 -> 57.5; kept 8 x 1: H2 S4096 (split 10 ways)
 // 33.8 against 49.5, H24 S2048 52.4 against 57.6.  D = 64: H8 S1024
 // 16.3 -> 10.6, H16 S2048 29.7 -> 24.6, kept H8 S4096 44.9 against 47.0.
-RowShape row_shape(const FlashParams& p, int D, int n_cu) {
-  const double T = (p.kv_end + kBKV - 1) / kBKV;
-  auto blocks = [&](int rows) {
-    return (int64_t)p.B * p.Hq * ((p.Sq + rows - 1) / rows);
-  };
+struct RowShape {
+  int r, g;
+};
+// `sp`: the split that 8 x 1 would take.  `key_groups`: whether the tiles may
+// be dealt to key groups.
+static RowShape row_shape(int64_t heads, int Sq, int kv_end, int D,
+                          const SplitPlan& sp, bool key_groups, int n_cu) {
+  const double T = (kv_end + kBKV - 1) / kBKV;
+  auto blocks = [&](int rows) { return heads * ((Sq + rows - 1) / rows); };
   const bool d64 = D == 64;
   // 8 x 1: whole rounds, then the last one (split or not)
   const double whole = d64 ? 8 + 0.95 * T : 9 + 1.6 * T;
   const int64_t n8 = blocks(256);
   double best;
-  if (p.ws != nullptr && p.n_split > 1) {
+  if (sp.n_split > 1) {
     const int64_t tail_rounds =
-        ((int64_t)p.n_tail * p.n_split + n_cu - 1) / n_cu;
-    best = (double)(p.n_main / n_cu) * whole +
-           (double)tail_rounds * ((d64 ? 0.95 : 1.6) * T / p.n_split) +
+        ((int64_t)sp.n_tail * sp.n_split + n_cu - 1) / n_cu;
+    best = (double)(sp.n_main / n_cu) * whole +
+           (double)tail_rounds * ((d64 ? 0.95 : 1.6) * T / sp.n_split) +
            (d64 ? 16 : 20);
   } else {
     best = (double)((n8 + n_cu - 1) / n_cu) * (n8 <= n_cu ? 0.9 : 1.0) * whole;
@@ -133,10 +137,39 @@ RowShape row_shape(const FlashParams& p, int D, int n_cu) {
   const double own = d64 ? 4.5 + 0.65 * T : 5.6 + 0.83 * T;
   const double shared = d64 ? 4.5 + 1.07 * T : 5.6 + 1.75 * T;
   consider((double)(per_cu / 2) * shared + (double)(per_cu % 2) * own, 4, 1);
-  if (!p.key_groups) return shape;
+  if (!key_groups) return shape;
   if (n4 <= n_cu) consider(d64 ? 6.0 + 0.46 * T : 7.5 + 0.72 * T, 4, 2);
   if (d64 && blocks(64) <= n_cu) consider(6.5 + 0.26 * T, 2, 4);
   return shape;
+}
+
+LaunchShape launch_shape(int B, int Hq, int Sq, int kv_end, int dim,
+                         LaunchForm form, size_t ws_bytes, int n_cu) {
+  const int D = kernel_dim(dim);
+  // (above head dim 128: 4 wavefronts, 32-key tiles)
+  const int bq = D == 256 ? 128 : kBQ, bkv = D == 256 ? 32 : kBKV;
+  const int64_t heads = (int64_t)B * Hq;
+  const int64_t n_wg = heads * ((Sq + bq - 1) / bq);
+  const int ntiles = (kv_end + bkv - 1) / bkv;
+  if (form == LaunchForm::kSingle) ws_bytes = 0;
+  if (D == 256) return {4, 1, split_plan(n_wg, ntiles, n_cu, D, bq, ws_bytes)};
+  auto shaped = [&](const SplitPlan& sp, bool key_groups) {
+    const RowShape w = row_shape(heads, Sq, kv_end, D, sp, key_groups, n_cu);
+    if (w.r == 8) return LaunchShape{8, 1, sp};
+    return LaunchShape{
+        w.r, w.g, SplitPlan{1, 0, (int)(heads * ((Sq + 32 * w.r - 1) / (32 * w.r))), 0}};
+  };
+  if (form == LaunchForm::kDense) {
+    // Smaller workgroups that beat 8 x 1 at its best split use no workspace:
+    // they are taken whatever the caller gave, so that a caller who asked how
+    // much the call uses, and gave none, gets them too.
+    const LaunchShape best =
+        shaped(split_plan(n_wg, ntiles, n_cu, D, bq), true);
+    if (best.r != 8 || best.split.ws_bytes <= ws_bytes) return best;
+  }
+  const SplitPlan sp = split_plan(n_wg, ntiles, n_cu, D, bq, ws_bytes);
+  if (form == LaunchForm::kTiles) return {8, 1, sp};
+  return shaped(sp, form == LaunchForm::kDense);
 }
 
 template <bool QK8, bool SPARSE>
@@ -145,15 +178,14 @@ static int launch_d128_v(const FlashParams& p, hipStream_t st) {
                          : launch_flash<FullDim<128>, QK8, SPARSE, false, 8, 1>(p, st);
 }
 
-int launch_flash_attn(const FlashParams& p, int D, hipStream_t st) {
-  int n_cu = 0;
-  if (int rc = device_cu_count(&n_cu)) return rc;
+int launch_flash_attn(const FlashParams& p, int D, const LaunchShape& shape,
+                      hipStream_t st) {
   if (D == 64) {
     if (p.k8 != nullptr || p.vt != nullptr || p.tile_span != nullptr)
       return set_error(DT_ERR_UNSUPPORTED,
                        "dt_flash_fwd: head dim 64 takes bf16 keys, row-major "
                        "V and no tile table");
-    return launch_dense<FullDim<64>, false>(p, n_cu, st);
+    return launch_dense<FullDim<64>, false>(p, shape, st);
   }
   const bool sparse = p.tile_span != nullptr;
   if (p.k8 != nullptr)
@@ -162,8 +194,8 @@ int launch_flash_attn(const FlashParams& p, int D, hipStream_t st) {
   if (sparse) return launch_d128_v<false, true>(p, st);
   // (packed and row-major V take the same shape: their results are equal
   // bit for bit)
-  return p.vt != nullptr ? launch_dense<FullDim<128>, true>(p, n_cu, st)
-                         : launch_dense<FullDim<128>, false>(p, n_cu, st);
+  return p.vt != nullptr ? launch_dense<FullDim<128>, true>(p, shape, st)
+                         : launch_dense<FullDim<128>, false>(p, shape, st);
 }
 
 }  // namespace dt

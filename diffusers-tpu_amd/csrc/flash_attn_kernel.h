@@ -1209,10 +1209,9 @@ int launch_flash(const FlashParams& base, hipStream_t st) {
   return DT_OK;
 }
 
-// A dense bf16 launch in the workgroup shape row_shape picks.
+// A dense bf16 launch in workgroups of shape `w`.
 template <class HD, bool VT>
-int launch_dense(const FlashParams& p, int n_cu, hipStream_t st) {
-  const RowShape w = row_shape(p, HD::D, n_cu);
+int launch_dense(const FlashParams& p, const LaunchShape& w, hipStream_t st) {
   if constexpr (HD::D == 64)
     if (w.r == 2) return launch_flash<HD, false, false, VT, 2, 4>(p, st);
   if (w.g == 2) return launch_flash<HD, false, false, VT, 4, 2>(p, st);

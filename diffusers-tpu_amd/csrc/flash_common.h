@@ -45,10 +45,6 @@ struct FlashParams {
   // n_tail = 0 when there is no split.
   float* ws;
   int n_main, n_split, n_tail;
-  // the tiles of a block may be dealt to key groups of one workgroup (their
-  // merge rounds as the tail split does; the entry points without a
-  // workspace argument keep one order of tiles)
-  bool key_groups;
   // o is stored past the caches: more than half of the 256 MB Infinity Cache,
   // it would only push out the K and V that the sweeps share (H40 Sq 48360
   // D = 64, 248 MB: Skv 128 196 -> 169 us, 512 357 -> 336; D = 128, 495 MB:
@@ -189,11 +185,14 @@ inline int ensure_lds_limit(const void* fn, int bytes,
   return DT_OK;
 }
 
+struct LaunchShape;
 // Launcher (flash_attn.hip): head dim D = 64 or 128.
-int launch_flash_attn(const FlashParams& p, int D, hipStream_t st);
+int launch_flash_attn(const FlashParams& p, int D, const LaunchShape& shape,
+                      hipStream_t st);
 // Launcher (flash_dims.hip): head dims p.dim below 128, multiples of 8 other
 // than 64; bf16 keys, row-major V, no tile table.
-int launch_flash_ragged(const FlashParams& p, hipStream_t st);
+int launch_flash_ragged(const FlashParams& p, const LaunchShape& shape,
+                        hipStream_t st);
 // Launcher (flash_wide.hip): head dims p.dim 136 to 256, bf16 keys, row-major
 // V, no tile table.
 int launch_flash_wide(const FlashParams& p, hipStream_t st);
@@ -212,11 +211,25 @@ SplitPlan split_plan(int64_t n_wg, int ntiles, int n_cu, int D, int bq,
                      size_t max_ws = ~size_t(0));
 int device_cu_count(int* n_cu);
 
-// Workgroup shape of a dense bf16 launch (flash_attn.hip): r row wavefronts
-// times g key groups.
-struct RowShape {
-  int r, g;
+// Channels of the kernel that runs head dim `dim` (a multiple of 8 up to 256).
+inline int kernel_dim(int dim) { return dim <= 64 ? 64 : dim <= 128 ? 128 : 256; }
+
+// How a call may be launched.
+enum class LaunchForm {
+  kDense,   // bf16 keys, every tile, a workspace argument: any shape, any split
+  kTiles,   // E4M3 keys or a tile table: 256-row blocks, split
+  kSingle,  // no workspace argument: one order of tiles, no split
 };
-RowShape row_shape(const FlashParams& p, int D, int n_cu);
+// What is launched: workgroups of r row wavefronts (32 query rows each) times
+// g key groups, and the split (whose ws_bytes is the workspace that is used).
+struct LaunchShape {
+  int r, g;
+  SplitPlan split;
+};
+// The launch of B * Hq heads of Sq query rows over kv_end keys, with at most
+// ws_bytes of workspace (flash_attn.hip).  The launches, the workspace query
+// and the plan queries all ask here.
+LaunchShape launch_shape(int B, int Hq, int Sq, int kv_end, int dim,
+                         LaunchForm form, size_t ws_bytes, int n_cu);
 
 }  // namespace dt

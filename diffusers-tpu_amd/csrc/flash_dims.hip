@@ -9,15 +9,14 @@
 
 namespace dt {
 
-int launch_flash_ragged(const FlashParams& p, hipStream_t st) {
-  int n_cu = 0;
-  if (int rc = device_cu_count(&n_cu)) return rc;
-  if (p.dim <= 48) return launch_dense<HeadDim<64, 3, true>, false>(p, n_cu, st);
-  if (p.dim < 64) return launch_dense<HeadDim<64, 4, true>, false>(p, n_cu, st);
-  if (p.dim <= 80) return launch_dense<HeadDim<128, 5, true>, false>(p, n_cu, st);
-  if (p.dim <= 96) return launch_dense<HeadDim<128, 6, true>, false>(p, n_cu, st);
-  if (p.dim <= 112) return launch_dense<HeadDim<128, 7, true>, false>(p, n_cu, st);
-  return launch_dense<HeadDim<128, 8, true>, false>(p, n_cu, st);
+int launch_flash_ragged(const FlashParams& p, const LaunchShape& shape,
+                        hipStream_t st) {
+  if (p.dim <= 48) return launch_dense<HeadDim<64, 3, true>, false>(p, shape, st);
+  if (p.dim < 64) return launch_dense<HeadDim<64, 4, true>, false>(p, shape, st);
+  if (p.dim <= 80) return launch_dense<HeadDim<128, 5, true>, false>(p, shape, st);
+  if (p.dim <= 96) return launch_dense<HeadDim<128, 6, true>, false>(p, shape, st);
+  if (p.dim <= 112) return launch_dense<HeadDim<128, 7, true>, false>(p, shape, st);
+  return launch_dense<HeadDim<128, 8, true>, false>(p, shape, st);
 }
 
 }  // namespace dt

@@ -24,26 +24,9 @@ static bool al16(const void* ptr) { return ((uintptr_t)ptr & 15u) == 0; }
 namespace dt {
 namespace {
 
-// The tail-split plan of a launch of B * Hq * ceil(Sq / 256) query blocks (128
-// rows at D = 256) over kv_end keys on the current device, within ws_bytes of
-// workspace;
-// dt_flash_fwd_ex, dt_flash_fwd_workspace_bytes and dt_flash_fwd_plan all
-// plan through here.
-int plan_launch(int B, int Hq, int Sq, int kv_end, int D, size_t ws_bytes,
-                int* n_cu, SplitPlan* sp) {
-  if (int rc = device_cu_count(n_cu)) return rc;
-  const int bq = D == 256 ? 128 : 256, bkv = D == 256 ? 32 : 64;
-  const int64_t n_wg = (int64_t)B * Hq * ((Sq + bq - 1) / bq);
-  *sp = split_plan(n_wg, (kv_end + bkv - 1) / bkv, *n_cu, D, bq, ws_bytes);
-  return DT_OK;
-}
-
-// Channels of the kernel that runs head dim D (a multiple of 8 up to 256).
-int kernel_dim(int D) { return D <= 64 ? 64 : D <= 128 ? 128 : 256; }
-
 // Validation and dispatch shared by dt_flash_fwd (bf16 keys),
 // dt_flash_fwd_qk8 (E4M3 keys, k_e4m3) and dt_flash_fwd_anydim (any_dim: head
-// dims no kernel is built for).
+// dims no kernel is built for).  has_ws: the entry point takes a workspace.
 int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
                 const uint16_t* v, uint16_t* o, int B, int Hq, int Hkv, int Sq,
                 int Skv, int D, const int64_t* q_strides,
@@ -53,7 +36,7 @@ int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
                 const int32_t* tile_ids, float* o32, float* m, float* l,
                 void* stream, const uint16_t* vt = nullptr,
                 int64_t vt_tiles = 0, void* ws = nullptr, size_t ws_bytes = 0,
-                const int32_t* kv_len_dev = nullptr, bool key_groups = false,
+                const int32_t* kv_len_dev = nullptr, bool has_ws = false,
                 bool any_dim = false) {
   const bool resid = (o32 != nullptr) || (m != nullptr) || (l != nullptr);
   const bool packed = vt != nullptr;
@@ -183,27 +166,27 @@ int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
   p.n_split = 1;
   p.n_tail = 0;
   p.n_main = 0;
-  p.key_groups = key_groups;
   p.nt_out = (int64_t)B * Hq * Sq * D * 2 > (128ll << 20);
   // (dt_flash_fwd_ex runs head dim 256 unsplit: the workspace is not used)
-  if (ws != nullptr && (D != 256 || any_dim)) {
-    if (!al16(ws))
-      return set_error(DT_ERR_UNSUPPORTED, "dt_flash_fwd_ex: misaligned workspace");
-    int n_cu = 0;
-    SplitPlan sp;
-    if (int rc = plan_launch(B, Hq, Sq, p.kv_end, kernel_dim(D), ws_bytes,
-                             &n_cu, &sp))
-      return rc;
-    if (sp.n_split > 1 && sp.ws_bytes <= ws_bytes) {
-      p.ws = (float*)ws;
-      p.n_split = sp.n_split;
-      p.n_tail = sp.n_tail;
-      p.n_main = sp.n_main;
-    }
+  const bool single = !has_ws || (D == 256 && !any_dim);
+  if (ws != nullptr && !single && !al16(ws))
+    return set_error(DT_ERR_UNSUPPORTED, "dt_flash_fwd_ex: misaligned workspace");
+  int n_cu = 0;
+  if (int rc = device_cu_count(&n_cu)) return rc;
+  const LaunchForm form = k_e4m3 || tile_span != nullptr ? LaunchForm::kTiles
+                          : single                       ? LaunchForm::kSingle
+                                                         : LaunchForm::kDense;
+  const LaunchShape shape = launch_shape(B, Hq, Sq, p.kv_end, D, form,
+                                         ws != nullptr ? ws_bytes : 0, n_cu);
+  if (shape.split.n_split > 1) {
+    p.ws = (float*)ws;
+    p.n_split = shape.split.n_split;
+    p.n_tail = shape.split.n_tail;
+    p.n_main = shape.split.n_main;
   }
   if (D > 128) return launch_flash_wide(p, st);
-  if (D != 64 && D != 128) return launch_flash_ragged(p, st);
-  return launch_flash_attn(p, D, st);
+  if (D != 64 && D != 128) return launch_flash_ragged(p, shape, st);
+  return launch_flash_attn(p, D, shape, st);
 }
 
 }  // namespace
@@ -274,11 +257,39 @@ extern "C" size_t dt_flash_fwd_anydim_workspace_bytes(int B, int Hq, int Sq,
     return 0;
   const int kv_end = (kv_len <= 0 || kv_len > Skv) ? Skv : kv_len;
   int n_cu = 0;
-  dt::SplitPlan sp;
-  if (dt::plan_launch(B, Hq, Sq, kv_end, dt::kernel_dim(D), ~size_t(0), &n_cu,
-                      &sp) != DT_OK)
-    return 0;
-  return sp.ws_bytes;
+  if (dt::device_cu_count(&n_cu) != DT_OK) return 0;
+  return dt::launch_shape(B, Hq, Sq, kv_end, D, dt::LaunchForm::kDense,
+                          ~size_t(0), n_cu).split.ws_bytes;
+}
+
+extern "C" int dt_flash_fwd_shape(int B, int Hq, int Sq, int Skv, int kv_len,
+                                  int D, int form, size_t workspace_bytes,
+                                  int compute_units, int32_t* shape,
+                                  size_t* ws_needed) {
+  if (shape == nullptr || ws_needed == nullptr)
+    return dt::set_error(DT_ERR_ARG, "dt_flash_fwd_shape: null output");
+  if (form < DT_FORM_DENSE || form > DT_FORM_SINGLE || compute_units < 0)
+    return dt::set_error(DT_ERR_ARG, "dt_flash_fwd_shape: form %d, %d CUs", form,
+                         compute_units);
+  if (D <= 0 || D % 8 || D > 256 || (form == DT_FORM_TILES && D != 128))
+    return dt::set_error(DT_ERR_UNSUPPORTED, "dt_flash_fwd_shape: head dim %d", D);
+  if (B <= 0 || Hq <= 0 || Sq <= 0 || Skv <= 0 || kv_len > Skv)
+    return dt::set_error(DT_ERR_SHAPE, "dt_flash_fwd_shape: bad shape");
+  const int kv_end = (kv_len <= 0) ? Skv : kv_len;
+  int n_cu = compute_units;
+  if (n_cu == 0)
+    if (int rc = dt::device_cu_count(&n_cu)) return rc;
+  const dt::LaunchShape s = dt::launch_shape(
+      B, Hq, Sq, kv_end, D, (dt::LaunchForm)form, workspace_bytes, n_cu);
+  const int rows = 32 * s.r, keys = D > 128 ? 32 : 64;
+  shape[0] = rows;
+  shape[1] = s.g;
+  shape[2] = (int32_t)((int64_t)B * Hq * ((Sq + rows - 1) / rows));
+  shape[3] = (kv_end + keys - 1) / keys;
+  shape[4] = s.split.n_split;
+  shape[5] = s.split.n_tail;
+  *ws_needed = s.split.ws_bytes;
+  return DT_OK;
 }
 
 extern "C" size_t dt_flash_fwd_workspace_bytes(int B, int Hq, int Sq, int Skv,
@@ -287,10 +298,9 @@ extern "C" size_t dt_flash_fwd_workspace_bytes(int B, int Hq, int Sq, int Skv,
     return 0;
   const int kv_end = (kv_len <= 0 || kv_len > Skv) ? Skv : kv_len;
   int n_cu = 0;
-  dt::SplitPlan sp;
-  if (dt::plan_launch(B, Hq, Sq, kv_end, D, ~size_t(0), &n_cu, &sp) != DT_OK)
-    return 0;
-  return sp.ws_bytes;
+  if (dt::device_cu_count(&n_cu) != DT_OK) return 0;
+  return dt::launch_shape(B, Hq, Sq, kv_end, D, dt::LaunchForm::kTiles,
+                          ~size_t(0), n_cu).split.ws_bytes;
 }
 
 extern "C" int dt_flash_fwd_plan(int B, int Hq, int Sq, int Skv, int kv_len,
@@ -319,18 +329,17 @@ extern "C" int dt_flash_fwd_plan(int B, int Hq, int Sq, int Skv, int kv_len,
     return DT_OK;
   }
   int n_cu = 0;
-  dt::SplitPlan sp;
-  if (int rc = dt::plan_launch(B, Hq, Sq, kv_end, D, workspace_bytes, &n_cu, &sp))
-    return rc;
-  const bool split = sp.n_split > 1 && sp.ws_bytes <= workspace_bytes;
-  const int64_t n_wg = (int64_t)B * Hq * ((Sq + 255) / 256);
+  if (int rc = dt::device_cu_count(&n_cu)) return rc;
+  const dt::SplitPlan sp =
+      dt::launch_shape(B, Hq, Sq, kv_end, D, dt::LaunchForm::kTiles,
+                       workspace_bytes, n_cu).split;
   plan[0] = n_cu;
-  plan[1] = (int32_t)n_wg;
+  plan[1] = (int32_t)((int64_t)B * Hq * ((Sq + 255) / 256));
   plan[2] = (kv_end + 63) / 64;
-  plan[3] = split ? sp.n_split : 1;
-  plan[4] = split ? sp.n_tail : 0;
-  plan[5] = split ? sp.n_main : (int32_t)n_wg;
-  *ws_needed = split ? sp.ws_bytes : 0;
+  plan[3] = sp.n_split;
+  plan[4] = sp.n_tail;
+  plan[5] = sp.n_main;
+  *ws_needed = sp.ws_bytes;
   return DT_OK;
 }
 

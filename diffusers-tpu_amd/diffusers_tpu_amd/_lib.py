@@ -21,6 +21,9 @@ DT_ERR_LAUNCH = -4
 
 ROPE_NONE, ROPE_HALF, ROPE_PAIR = 0, 1, 2
 
+# dt_form: how a call may be launched
+FORM_DENSE, FORM_TILES, FORM_SINGLE = 0, 1, 2
+
 # most parts of one dt_merge_residuals call (DT_MERGE_MAX_PARTS)
 MERGE_MAX_PARTS = 16
 
@@ -73,6 +76,7 @@ SIGNATURES = {
     "dt_flash_fwd_anydim": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P,
                                  _P, _P, _P, _F, _I, _P, _P, _P, _P, _P, _P,
                                  _Z, _P]),
+    "dt_flash_fwd_shape": (_I, [_I, _I, _I, _I, _I, _I, _I, _Z, _I, _P, _P]),
     "dt_flash_fwd_anydim_workspace_bytes": (_Z, [_I, _I, _I, _I, _I, _I]),
     "dt_merge_residuals": (_I, [_P, _P, _P, _I, _L, _I, _P, _P]),
 }

@@ -11,8 +11,8 @@ and 64 keys per stage.  What a shape decides here is the launch plan: how
 the query blocks of a partly filled last round of workgroups are split
 over their key tiles (``launch_plan``, from ``dt_flash_fwd_plan``, the
 planner ``dt_flash_fwd_ex`` itself uses).  Dense bf16 calls with few query
-blocks or few key tiles run in smaller row blocks instead, which the plan does
-not describe.
+blocks or few key tiles run in smaller row blocks instead; ``launch_shape``
+says what ``attention`` launches for a shape.
 
 The reference's entry points keep their names, arguments and resolution
 order (pinned, else tuned, else default), so callers that resolve blocks
@@ -177,7 +177,7 @@ def rank_block_candidates(seq_len: int, head_dim: int = 128,
 
 @dataclasses.dataclass(frozen=True)
 class LaunchPlan:
-  """What ``dt_flash_fwd_ex`` runs for a shape on the current device.
+  """The plan of 256-row blocks for a shape on the current device.
 
   Attributes:
     compute_units: CUs of the device (workgroups per round).
@@ -204,13 +204,13 @@ def launch_plan(batch: int, heads: int, seq_len: int,
                 kv_seq_len: int | None = None, head_dim: int = 128, *,
                 kv_len: int | None = None, qk_fp8: bool = False,
                 workspace_bytes: int | None = None) -> LaunchPlan:
-  """The launch plan of one attention call on the current GPU.
+  """The plan of 256-row blocks of one attention call on the current GPU (what
+  ``dt_flash_fwd_plan`` answers), which calls with ``qk_fp8`` or a tile table
+  follow; ``launch_shape`` describes the others.
 
   ``workspace_bytes``: the workspace the call would pass (None: as much as
-  the best plan uses, which is what ``attention`` allocates at head dims 64
-  and 128).  Other head dims plan here as the next of 64, 128 and 256 (with
-  ``qk_fp8`` they run so, zero-padded).  ``attention`` itself runs the others
-  at their own width, and splits above 128 too, where this plan has no split.
+  the best plan uses).  Other head dims plan here as the next of 64, 128 and
+  256, the last unsplit.
   """
   from diffusers_tpu_amd import _lib
   from diffusers_tpu_amd.kernels.splash import kernel_head_dim
@@ -236,3 +236,54 @@ def launch_plan(batch: int, heads: int, seq_len: int,
                     key_tiles=plan[2], rounds=plan[1] / plan[0],
                     split_parts=plan[3], tail_blocks=plan[4],
                     whole_blocks=plan[5], workspace_bytes=need.value)
+
+
+@dataclasses.dataclass(frozen=True)
+class LaunchShape:
+  """What ``attention`` launches for a shape.
+
+  Attributes:
+    block_rows: query rows of a workgroup (256, 128 or 64).
+    key_groups: groups of a workgroup's wavefronts its key tiles are dealt to.
+    query_blocks: B * H * ceil(Sq / block_rows).
+    key_tiles: key tiles each block sweeps (64 keys; 32 above head dim 128).
+    split_parts: parts each tail block runs as (1: no split).
+    tail_blocks: query blocks of the last round that are split.
+    workspace_bytes: workspace the call uses.
+  """
+
+  block_rows: int
+  key_groups: int
+  query_blocks: int
+  key_tiles: int
+  split_parts: int
+  tail_blocks: int
+  workspace_bytes: int
+
+
+def launch_shape(batch: int, heads: int, seq_len: int,
+                 kv_seq_len: int | None = None, head_dim: int = 128, *,
+                 kv_len: int | None = None, qk_fp8: bool = False,
+                 tile_table: bool = False, workspace_bytes: int | None = None,
+                 compute_units: int = 0) -> LaunchShape:
+  """What one attention call launches (``dt_flash_fwd_shape``) on the current
+  GPU, or on one of ``compute_units`` CUs (then no GPU is needed).
+
+  ``kv_len``: a host length (None for a length on the GPU).  ``tile_table``:
+  a block-sparse call.  ``workspace_bytes``: the most workspace there is
+  (None: as much as the call uses).
+  """
+  from diffusers_tpu_amd import _lib
+  if head_dim % 8 or head_dim > (128 if qk_fp8 or tile_table else 256):
+    raise NotImplementedError(f"head_dim {head_dim}")
+  tiles = qk_fp8 or tile_table  # (these run zero-padded to 128)
+  shape = (ctypes.c_int32 * 6)()
+  need = ctypes.c_size_t(0)
+  limit = ctypes.c_size_t(-1).value if workspace_bytes is None else \
+      int(workspace_bytes)
+  _lib.check("dt_flash_fwd_shape", _lib.load().dt_flash_fwd_shape(
+      batch, heads, seq_len, seq_len if kv_seq_len is None else kv_seq_len,
+      0 if kv_len is None else int(kv_len), 128 if tiles else head_dim,
+      _lib.FORM_TILES if tiles else _lib.FORM_DENSE, limit, compute_units,
+      shape, ctypes.byref(need)))
+  return LaunchShape(*shape, workspace_bytes=need.value)

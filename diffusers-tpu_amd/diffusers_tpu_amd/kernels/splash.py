@@ -173,9 +173,11 @@ class AttentionWorkspace:
     return self._get("_split", (nbytes + 3) // 4, torch.float32)
 
   def reserve(self, query_shape, key_shape, kv_len=None, *, packed=None):
-    """Allocates what a call with these shapes needs (``kv_len`` an int or
-    ``None``; a device length plans for every key).  ``packed``: whether
-    the call streams packed V (default: as ``attention`` decides)."""
+    """Allocates what a call with these shapes needs in any form (``kv_len``
+    an int or ``None``; a device length plans for every key): the split of
+    256-row blocks, also where the bf16 call runs in smaller workgroups and
+    leaves it to calls with ``qk_fp8``.  ``packed``: whether the call streams
+    packed V (default: as ``attention`` decides)."""
     b, hq, sq, d = query_shape
     _, hkv, skv, _ = key_shape
     # a device length, or per-sample lengths: plan for every key
@@ -185,8 +187,9 @@ class AttentionWorkspace:
     if packed:
       self.packed_v(packed_v_numel(b, hkv, n))
     with _lib.device_guard(self.device.index):
-      nbytes = _lib.load().dt_flash_fwd_anydim_workspace_bytes(
-          b, hq, sq, skv, 0 if n == skv else n, d)
+      nbytes = _split_bytes(b, hq, sq, skv, 0 if n == skv else n,
+                            d if d > 128 else kernel_head_dim(d),
+                            self.device.index, tiles=d <= 128)
     if nbytes:
       self.split(nbytes)
     return self
@@ -461,11 +464,15 @@ def _call_anydim(query, key, value, scale, n, out, residual, mk, workspace):
 
 
 @functools.lru_cache(maxsize=4096)
-def _split_bytes(b, hq, sq, skv, n, d, device_index):
-  """``dt_flash_fwd_anydim_workspace_bytes`` (at head dims 64 and 128 the
-  bytes ``dt_flash_fwd_ex`` uses) per shape and device, queried once (the
-  current device is ``device_index`` when it is called)."""
-  return _lib.load().dt_flash_fwd_anydim_workspace_bytes(b, hq, sq, skv, n, d)
+def _split_bytes(b, hq, sq, skv, n, d, device_index, tiles=False):
+  """Workspace bytes per shape and device, queried once (the current device
+  is ``device_index`` when it is called): of a dense bf16 call
+  (``dt_flash_fwd_anydim_workspace_bytes``), or with ``tiles`` of one with
+  E4M3 keys or a tile table (``dt_flash_fwd_workspace_bytes``)."""
+  lib = _lib.load()
+  fn = lib.dt_flash_fwd_workspace_bytes if tiles else \
+      lib.dt_flash_fwd_anydim_workspace_bytes
+  return fn(b, hq, sq, skv, n, d)
 
 
 def _call_ex(q, k, k_format, v, packed_v, out, residual, hkv, skv, scale, n,
@@ -494,7 +501,8 @@ def _call_ex(q, k, k_format, v, packed_v, out, residual, hkv, skv, scale, n,
           (b, hq, sq, d), device=q.device, dtype=torch.bfloat16)
       outs = (o.data_ptr(), s3(o), None, None, None)
     nbytes = _split_bytes(b, hq, sq, skv, 0 if n_dev is not None else n_host,
-                          d, q.device.index)
+                          d, q.device.index,
+                          tiles=k_format == 1 or span is not None)
     if not nbytes:
       ws = None
     elif workspace is not None:

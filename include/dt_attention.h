@@ -42,6 +42,8 @@
  *   dt_merge_residuals — the LSE-space merge of residual outputs from key
  *                      shards (kernels/splash.py:653-664).
  *   dt_flash_fwd_plan — the launch plan (grid, tail split) of a shape.
+ *   dt_flash_fwd_shape — what a call of a shape launches (rows of a workgroup,
+ *                      key groups, tail split).
  *   dt_flash_fwd_ex_noalloc — dt_flash_fwd_ex with its workspace in static
  *                      device memory (no reference counterpart: for
  *                      callers that cannot allocate).
@@ -441,7 +443,11 @@ int dt_flash_fwd_anydim(const uint16_t* q, const uint16_t* k,
                         const int32_t* kv_len_dev, const float* mk, float* o32,
                         float* m, float* l, void* workspace,
                         size_t workspace_bytes, void* stream);
-/* Workspace bytes dt_flash_fwd_anydim can use (as the function above). */
+/*
+ * Workspace bytes that a dense bf16 call uses: dt_flash_fwd_anydim, or
+ * dt_flash_fwd_ex at head dim 64 or 128 without a tile table.  0 where it runs
+ * in smaller workgroups instead of splitting (dt_flash_fwd_shape).
+ */
 size_t dt_flash_fwd_anydim_workspace_bytes(int B, int Hq, int Sq, int Skv,
                                            int kv_len, int D);
 
@@ -457,13 +463,34 @@ size_t dt_flash_fwd_anydim_workspace_bytes(int B, int Hq, int Sq, int Skv,
  * and never splits.  This is the gfx950 side of the reference's per-shape block
  * resolution (kernels/block_sizes.py:537-577, used at
  * kernels/mesh_attention.py:198-215): the tile is fixed, and what a shape
- * decides is the tail split.  A dense bf16 call with few query blocks or few
- * key tiles may run in workgroups of 128 or 64 rows instead and leave the
- * workspace unused.
+ * decides is the tail split.  It is the plan of 256-row blocks, which calls
+ * with E4M3 keys or a tile table always follow; what a dense bf16 call with few
+ * query blocks or few key tiles runs instead, dt_flash_fwd_shape says.
  */
 int dt_flash_fwd_plan(int B, int Hq, int Sq, int Skv, int kv_len, int D,
                       size_t workspace_bytes, int32_t* plan,
                       size_t* ws_needed);
+
+/*
+ * What a call of this shape launches, given workspace_bytes of workspace, on a
+ * device of compute_units CUs (0: the current device).  form: one of dt_form.
+ * shape[6] receives: [0] the query rows of a workgroup (256, 128 or 64), [1]
+ * the key groups its tiles are dealt to (their results merged in LDS), [2] the
+ * query blocks (B * Hq * ceil(Sq / rows)), [3] the key tiles per block (64
+ * keys; 32 above head dim 128), [4] the parts each tail block is split into
+ * (1: no split), [5] the tail blocks split; *ws_needed the workspace bytes
+ * used.  D: a multiple of 8 up to 256.  Pass kv_len 0 for calls that give
+ * kv_len_dev.  With compute_units > 0 no device is needed.
+ */
+enum dt_form {
+  DT_FORM_DENSE = 0,  /* dt_flash_fwd_anydim; dt_flash_fwd_ex at head dim 64 or
+                         128 with bf16 keys and no tile table */
+  DT_FORM_TILES = 1,  /* E4M3 keys or a tile table (head dim 128) */
+  DT_FORM_SINGLE = 2  /* dt_flash_fwd; dt_flash_fwd_ex at head dim 256 */
+};
+int dt_flash_fwd_shape(int B, int Hq, int Sq, int Skv, int kv_len, int D,
+                       int form, size_t workspace_bytes, int compute_units,
+                       int32_t* shape, size_t* ws_needed);
 
 /*
  * dt_flash_fwd_ex without a workspace argument: the tail split's partial

@@ -1,0 +1,80 @@
+"""Every workgroup shape of the dense bf16 kernel at every kernel width, the
+shape that runs asserted: against the float64 oracle, with per-sample lengths
+that end inside a tile and that leave key groups and split parts without tiles,
+and packed V against row-major V bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_helpers import assert_attn_close, banner, seeded, to64
+from oracle import attention as A
+
+pytestmark = pytest.mark.gpu
+
+# (rows, key groups, split): (B, H, Sq, Skv) on 256 CUs
+NARROW = {(64, 4, False): (2, 1, 130, 700), (128, 1, False): (2, 2, 130, 130),
+          (128, 2, False): (2, 40, 200, 700), (256, 1, False): (2, 22, 700, 1087),
+          (256, 1, True): (2, 1, 200, 6000)}
+FULL = {(128, 1, False): (2, 2, 200, 130), (128, 2, False): (2, 1, 200, 1500),
+        (256, 1, False): (2, 22, 700, 700), (256, 1, True): (2, 1, 200, 3000)}
+CASES = [(d, want, size) for dims, table in (((40, 56, 64), NARROW),
+                                             ((72, 88, 104, 120, 128), FULL))
+         for d in dims for want, size in table.items()]
+
+
+@pytest.fixture(scope="module")
+def sp():
+  if not torch.cuda.is_available():
+    pytest.skip("no GPU")
+  if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+    pytest.skip("the sizes choose their shapes on 256 CUs")
+  from diffusers_tpu_amd.kernels import splash
+  return splash
+
+
+@pytest.mark.parametrize("d,want,size", CASES,
+                         ids=[f"{d}-{w}" for d, w, _ in CASES])
+def test_shape_matches_oracle(sp, d, want, size):
+  from diffusers_tpu_amd.kernels.block_sizes import launch_shape
+  banner(f"shape {want} dim {d} {size}")
+  b, h, sq, skv = size
+  s = launch_shape(b, h, sq, skv, d)
+  assert (s.block_rows, s.key_groups, s.split_parts > 1) == want
+  assert sp._split_bytes(b, h, sq, skv, 0, d, 0) == s.workspace_bytes
+  q, k, v = (seeded((b, h, n, d), 700 + i) for i, n in enumerate((sq, skv, skv)))
+  heads = sorted({0, h - 1})
+  rows = np.unique(np.r_[0:40, 120:136, max(0, sq - 70):sq])
+  rows = rows[rows < sq]
+  for lens in (None, (skv - 29, 50)):
+    n = None if lens is None else torch.tensor(lens, device="cuda",
+                                               dtype=torch.int32)
+    got = sp.attention(q, k, v, kv_len=n)
+    o, m, l = sp.residual_attention(q, k, v, kv_len=n)
+    for i in range(b):
+      w = A.attention_f64(to64(q[i:i + 1, heads][:, :, rows]),
+                          to64(k[i:i + 1, heads]), to64(v[i:i + 1, heads]),
+                          kv_len=skv if lens is None else lens[i])
+      pick = lambda t: to64(t[i:i + 1, heads][:, :, rows])
+      assert_attn_close(pick(got), w, f"{lens} sample {i}")
+      assert_attn_close(pick(o) / pick(l), w, f"{lens} residual {i}")
+    if d == 128:
+      packed = sp.pack_v(v, n)
+      assert torch.equal(sp._launch(q, k, v, None, n, packed_v=packed), got)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_smaller_workgroups_take_no_workspace(sp, d):
+  """Calls that run in smaller workgroups leave a caller's workspace empty;
+  reserve still covers every form of a call of the shape."""
+  banner(f"workspace of small shapes, dim {d}")
+  q = seeded((1, 8, 500, d), 710)
+  ws = sp.AttentionWorkspace()
+  want = sp.attention(q, q, q)
+  assert torch.equal(sp.attention(q, q, q, workspace=ws), want)
+  assert ws._split is None
+  ws.reserve(q.shape, q.shape)
+  held = ws._split
+  assert held is not None
+  if d == 128:
+    sp.attention(q, q, q, qk_fp8=True, workspace=ws)
+    assert ws._split is held

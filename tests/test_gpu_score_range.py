@@ -62,7 +62,11 @@ MASKED = [(2, 22, 250, 1500, 128), (1, 8, 1000, 1024, 64), (1, 24, 300, 1500, 72
 def test_masked_tiles_after_the_first(dta, case, low):
   """All keys but tile 0 and a few of the last ones masked by a channel."""
   b, h, sq, skv, d = case
+  from diffusers_tpu_amd.kernels.block_sizes import launch_shape
   banner(f"masked tiles {case} {low}")
+  if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+    s = launch_shape(b, h, sq, skv, d)
+    assert s.key_groups > 1 if d <= 128 else s.split_parts > 1
   q, k, v = _inputs(b, h, sq, skv, d, 660)
   q[..., 0], k[..., 0] = 1.0, 0.0
   keep = np.r_[0:64, skv - 5:skv]

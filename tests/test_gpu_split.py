@@ -85,7 +85,11 @@ CASES = [
     (1, 2, 2, 300, 4096, None),       # 4 blocks -> 8 parts each
     (2, 4, 2, 700, 3000, 2901),       # GQA, kv_len mid-tile
     (1, 3, 3, 256, 520, None),        # few tiles: ragged part sizes
+    # (the first and the last run in smaller workgroups, whole; these split)
+    (2, 2, 1, 300, 6000, 5901, 64),
+    (1, 3, 3, 256, 2100, None),
 ]
+SPLIT = [c for i, c in enumerate(CASES) if i not in (0, 3)]
 
 
 @pytest.mark.parametrize("case", CASES)
@@ -128,6 +132,32 @@ def test_split_matches_unsplit_and_oracle(sp, case):
   lse = gm + np.log2(to64(l))
   np.testing.assert_allclose(lse, to64(rm) + np.log2(to64(rl)), atol=3e-3,
                              rtol=0)
+
+
+def test_cases_that_split(sp):
+  from diffusers_tpu_amd.kernels.block_sizes import launch_shape
+  banner("split cases")
+  if _cus() != 256:
+    pytest.skip("the sizes choose their split on 256 CUs")
+  for case in CASES:
+    b, hq, hkv, sq, skv, kv_len = case[:6]
+    s = launch_shape(b, hq, sq, skv, case[6] if len(case) > 6 else 128,
+                     kv_len=kv_len)
+    assert (s.split_parts > 1) == (case in SPLIT), case
+    assert (s.block_rows == 256) == (case in SPLIT), case
+
+
+def test_split_few_tiles(sp):
+  """E4M3 calls keep 256-row blocks: 9 tiles in 3 parts."""
+  from diffusers_tpu_amd.kernels.block_sizes import launch_shape
+  from diffusers_tpu_amd.kernels.fp8_cast import quantize_saturating
+  banner("split E4M3, few tiles")
+  q, k, v = (seeded((1, 3, n, 128), 186 + i)
+             for i, n in enumerate((256, 520, 520)))
+  assert launch_shape(1, 3, 256, 520, qk_fp8=True).split_parts > 1
+  got = sp._launch(q, k, v, None, None, qk_fp8=True)
+  ref = _nosplit(sp, q, quantize_saturating(k), v, None, False, k_format=1)
+  assert (got.float() - ref.float()).abs().max().item() <= 2 ** -7
 
 
 def test_split_qk8_fixed_m_and_sparse(sp):
