@@ -151,25 +151,23 @@ LaunchShape launch_shape(int B, int Hq, int Sq, int kv_end, int dim,
   const int64_t heads = (int64_t)B * Hq;
   const int64_t n_wg = heads * ((Sq + bq - 1) / bq);
   const int ntiles = (kv_end + bkv - 1) / bkv;
-  if (form == LaunchForm::kSingle) ws_bytes = 0;
   if (D == 256) return {4, 1, split_plan(n_wg, ntiles, n_cu, D, bq, ws_bytes)};
   auto shaped = [&](const SplitPlan& sp, bool key_groups) {
     const RowShape w = row_shape(heads, Sq, kv_end, D, sp, key_groups, n_cu);
     if (w.r == 8) return LaunchShape{8, 1, sp};
-    return LaunchShape{
-        w.r, w.g, SplitPlan{1, 0, (int)(heads * ((Sq + 32 * w.r - 1) / (32 * w.r))), 0}};
+    const int64_t blocks = heads * ((Sq + 32 * w.r - 1) / (32 * w.r));
+    return LaunchShape{w.r, w.g, SplitPlan{1, 0, (int)blocks, w.g > 1 ? kGroupsWs : 0}};
   };
   if (form == LaunchForm::kDense) {
-    // Smaller workgroups that beat 8 x 1 at its best split use no workspace:
-    // they are taken whatever the caller gave, so that a caller who asked how
-    // much the call uses, and gave none, gets them too.
+    // (the best of all, where the workspace allows it: a caller who gives what
+    // the query says gets it)
     const LaunchShape best =
         shaped(split_plan(n_wg, ntiles, n_cu, D, bq), true);
-    if (best.r != 8 || best.split.ws_bytes <= ws_bytes) return best;
+    if (best.split.ws_bytes <= ws_bytes) return best;
   }
   const SplitPlan sp = split_plan(n_wg, ntiles, n_cu, D, bq, ws_bytes);
   if (form == LaunchForm::kTiles) return {8, 1, sp};
-  return shaped(sp, form == LaunchForm::kDense);
+  return shaped(sp, ws_bytes >= kGroupsWs);
 }
 
 template <bool QK8, bool SPARSE>

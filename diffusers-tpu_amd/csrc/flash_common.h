@@ -216,12 +216,15 @@ inline int kernel_dim(int dim) { return dim <= 64 ? 64 : dim <= 128 ? 128 : 256;
 
 // How a call may be launched.
 enum class LaunchForm {
-  kDense,   // bf16 keys, every tile, a workspace argument: any shape, any split
-  kTiles,   // E4M3 keys or a tile table: 256-row blocks, split
-  kSingle,  // no workspace argument: one order of tiles, no split
+  kDense,  // bf16 keys, every tile: any shape, any split
+  kTiles,  // E4M3 keys or a tile table: 256-row blocks, split
 };
+// The least workspace that allows key groups, though they use none of it: a
+// call without a workspace keeps one order of tiles (dt_flash_fwd's bits).
+constexpr size_t kGroupsWs = 16;
 // What is launched: workgroups of r row wavefronts (32 query rows each) times
-// g key groups, and the split (whose ws_bytes is the workspace that is used).
+// g key groups, and the split, whose ws_bytes is the workspace it takes
+// (kGroupsWs with key groups).
 struct LaunchShape {
   int r, g;
   SplitPlan split;

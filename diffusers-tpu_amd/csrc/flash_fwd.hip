@@ -26,7 +26,7 @@ namespace {
 
 // Validation and dispatch shared by dt_flash_fwd (bf16 keys),
 // dt_flash_fwd_qk8 (E4M3 keys, k_e4m3) and dt_flash_fwd_anydim (any_dim: head
-// dims no kernel is built for).  has_ws: the entry point takes a workspace.
+// dims no kernel is built for).
 int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
                 const uint16_t* v, uint16_t* o, int B, int Hq, int Hkv, int Sq,
                 int Skv, int D, const int64_t* q_strides,
@@ -36,8 +36,7 @@ int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
                 const int32_t* tile_ids, float* o32, float* m, float* l,
                 void* stream, const uint16_t* vt = nullptr,
                 int64_t vt_tiles = 0, void* ws = nullptr, size_t ws_bytes = 0,
-                const int32_t* kv_len_dev = nullptr, bool has_ws = false,
-                bool any_dim = false) {
+                const int32_t* kv_len_dev = nullptr, bool any_dim = false) {
   const bool resid = (o32 != nullptr) || (m != nullptr) || (l != nullptr);
   const bool packed = vt != nullptr;
   if (!q || !k || !q_strides || !k_strides ||
@@ -168,16 +167,15 @@ int flash_entry(const uint16_t* q, const void* k, bool k_e4m3,
   p.n_main = 0;
   p.nt_out = (int64_t)B * Hq * Sq * D * 2 > (128ll << 20);
   // (dt_flash_fwd_ex runs head dim 256 unsplit: the workspace is not used)
-  const bool single = !has_ws || (D == 256 && !any_dim);
-  if (ws != nullptr && !single && !al16(ws))
+  if (ws == nullptr || (D == 256 && !any_dim)) ws_bytes = 0;
+  if (ws_bytes > 0 && !al16(ws))
     return set_error(DT_ERR_UNSUPPORTED, "dt_flash_fwd_ex: misaligned workspace");
   int n_cu = 0;
   if (int rc = device_cu_count(&n_cu)) return rc;
   const LaunchForm form = k_e4m3 || tile_span != nullptr ? LaunchForm::kTiles
-                          : single                       ? LaunchForm::kSingle
                                                          : LaunchForm::kDense;
-  const LaunchShape shape = launch_shape(B, Hq, Sq, p.kv_end, D, form,
-                                         ws != nullptr ? ws_bytes : 0, n_cu);
+  const LaunchShape shape =
+      launch_shape(B, Hq, Sq, p.kv_end, D, form, ws_bytes, n_cu);
   if (shape.split.n_split > 1) {
     p.ws = (float*)ws;
     p.n_split = shape.split.n_split;
@@ -247,7 +245,7 @@ extern "C" int dt_flash_fwd_anydim(
   return dt::flash_entry(q, k, false, v, o, B, Hq, Hkv, Sq, Skv, D, q_strides,
                          k_strides, v_strides, o_strides, scale, kv_len, mk,
                          nullptr, nullptr, o32, m, l, stream, nullptr, 0,
-                         workspace, workspace_bytes, kv_len_dev, true, true);
+                         workspace, workspace_bytes, kv_len_dev, true);
 }
 
 extern "C" size_t dt_flash_fwd_anydim_workspace_bytes(int B, int Hq, int Sq,
@@ -268,7 +266,7 @@ extern "C" int dt_flash_fwd_shape(int B, int Hq, int Sq, int Skv, int kv_len,
                                   size_t* ws_needed) {
   if (shape == nullptr || ws_needed == nullptr)
     return dt::set_error(DT_ERR_ARG, "dt_flash_fwd_shape: null output");
-  if (form < DT_FORM_DENSE || form > DT_FORM_SINGLE || compute_units < 0)
+  if ((form != DT_FORM_DENSE && form != DT_FORM_TILES) || compute_units < 0)
     return dt::set_error(DT_ERR_ARG, "dt_flash_fwd_shape: form %d, %d CUs", form,
                          compute_units);
   if (D <= 0 || D % 8 || D > 256 || (form == DT_FORM_TILES && D != 128))
@@ -426,5 +424,5 @@ extern "C" int dt_flash_fwd_ex(
   return dt::flash_entry(q, k, k_format == 1, v, o, B, Hq, Hkv, Sq, Skv, D,
                          q_strides, k_strides, v_strides, o_strides, scale,
                          kv_len, mk, tile_span, tile_ids, o32, m, l, stream, vt,
-                         vt_tiles, workspace, workspace_bytes, kv_len_dev, true);
+                         vt_tiles, workspace, workspace_bytes, kv_len_dev);
 }

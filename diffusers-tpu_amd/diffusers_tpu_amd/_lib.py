@@ -22,7 +22,7 @@ DT_ERR_LAUNCH = -4
 ROPE_NONE, ROPE_HALF, ROPE_PAIR = 0, 1, 2
 
 # dt_form: how a call may be launched
-FORM_DENSE, FORM_TILES, FORM_SINGLE = 0, 1, 2
+FORM_DENSE, FORM_TILES = 0, 1
 
 # most parts of one dt_merge_residuals call (DT_MERGE_MAX_PARTS)
 MERGE_MAX_PARTS = 16

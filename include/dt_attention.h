@@ -404,8 +404,10 @@ int dt_pack_v(const uint16_t* v, uint16_t* vt, int B, int Hkv, int Skv, int D,
  * part rounds its probabilities to bf16 against its own reference m, so
  * results differ from the unsplit ones at bf16 rounding level.  The
  * workspace is scratch for the duration of the call on `stream`; calls that
- * share one workspace must be ordered.  null: no split.  No element of it
- * needs initializing.
+ * share one workspace must be ordered.  No element of it needs initializing.
+ * With at least 16 bytes a dense bf16 call may also deal the tiles of a block
+ * to key groups of one workgroup, which rounds as the split does and uses none
+ * of it.  null: neither; the results are those of dt_flash_fwd bit for bit.
  */
 int dt_flash_fwd_ex(const uint16_t* q, const void* k, int k_format,
                     const uint16_t* v, const int64_t* v_strides,
@@ -445,8 +447,9 @@ int dt_flash_fwd_anydim(const uint16_t* q, const uint16_t* k,
                         size_t workspace_bytes, void* stream);
 /*
  * Workspace bytes that a dense bf16 call uses: dt_flash_fwd_anydim, or
- * dt_flash_fwd_ex at head dim 64 or 128 without a tile table.  0 where it runs
- * in smaller workgroups instead of splitting (dt_flash_fwd_shape).
+ * dt_flash_fwd_ex at head dim 64 or 128 without a tile table.  Where it runs in
+ * smaller workgroups instead of splitting (dt_flash_fwd_shape), 16 with key
+ * groups and 0 without.
  */
 size_t dt_flash_fwd_anydim_workspace_bytes(int B, int Hq, int Sq, int Skv,
                                            int kv_len, int D);
@@ -483,10 +486,9 @@ int dt_flash_fwd_plan(int B, int Hq, int Sq, int Skv, int kv_len, int D,
  * kv_len_dev.  With compute_units > 0 no device is needed.
  */
 enum dt_form {
-  DT_FORM_DENSE = 0,  /* dt_flash_fwd_anydim; dt_flash_fwd_ex at head dim 64 or
-                         128 with bf16 keys and no tile table */
-  DT_FORM_TILES = 1,  /* E4M3 keys or a tile table (head dim 128) */
-  DT_FORM_SINGLE = 2  /* dt_flash_fwd; dt_flash_fwd_ex at head dim 256 */
+  DT_FORM_DENSE = 0, /* bf16 keys, no tile table (dt_flash_fwd_ex at head dim
+                        256 launches as with no workspace) */
+  DT_FORM_TILES = 1  /* E4M3 keys or a tile table (head dim 128) */
 };
 int dt_flash_fwd_shape(int B, int Hq, int Sq, int Skv, int kv_len, int D,
                        int form, size_t workspace_bytes, int compute_units,
@@ -505,7 +507,7 @@ int dt_flash_fwd_shape(int B, int Hq, int Sq, int Skv, int kv_len, int D,
  * scratch the call may use, exactly as if dt_flash_fwd_ex were given a
  * workspace of that many bytes (same split, bit-identical results);
  * dt_flash_fwd_workspace_bytes(...) gives the best split's need, 0 means
- * no split.  scratch_bytes above DT_NOALLOC_SCRATCH_BYTES is rejected
+ * no workspace.  scratch_bytes above DT_NOALLOC_SCRATCH_BYTES is rejected
  * (DT_ERR_ARG).  Nothing in the scratch needs to start at zero.  Every
  * call on one GPU shares that GPU's scratch, which keeps the last call's
  * contents: calls that overlap on one GPU (other streams, other threads)

@@ -14,7 +14,7 @@ def shape(*args, **kw):
 def test_shapes_of_the_models_layers():
   s = shape(1, 8, 1024, head_dim=64)       # plumbing layer: 4 key groups
   assert (s.block_rows, s.key_groups, s.split_parts) == (64, 4, 1)
-  assert (s.query_blocks, s.key_tiles, s.workspace_bytes) == (128, 16, 0)
+  assert (s.query_blocks, s.key_tiles, s.workspace_bytes) == (128, 16, 16)
   s = shape(2, 24, 512)                    # text refiner: 128-row blocks
   assert (s.block_rows, s.key_groups, s.workspace_bytes) == (128, 1, 0)
   s = shape(1, 40, 48360, 512)             # cross-attention
@@ -29,21 +29,22 @@ def test_shapes_of_the_models_layers():
 
 
 @pytest.mark.parametrize("d", [8, 40, 64, 72, 104, 128, 136, 256])
-def test_no_workspace_gives_the_shape_of_a_call_that_needs_none(d):
-  """A call whose best launch uses no workspace launches the same without."""
+def test_workspace_limits(d):
+  """What a call takes is enough for it; with less it splits into fewer parts
+  or not at all, and without any it keeps one order of tiles."""
   for b, h, sq, skv in [(1, 1, 1, 1), (1, 8, 1024, 1024), (2, 24, 512, 512),
                         (1, 3, 700, 1500), (1, 40, 9000, 512),
                         (2, 22, 700, 700), (1, 2, 300, 4096)]:
     s = shape(b, h, sq, skv, d)
     assert s.query_blocks == b * h * -(-sq // s.block_rows)
-    assert (s.workspace_bytes > 0) == (s.split_parts > 1)
-    if d <= 128 and s.block_rows < 256:
-      assert s.split_parts == 1
-    if not s.workspace_bytes:
-      assert s == shape(b, h, sq, skv, d, workspace_bytes=0)
+    if s.block_rows < 256 and d <= 128:
+      assert (s.split_parts, s.workspace_bytes) == (1, 16 * (s.key_groups > 1))
     else:
-      assert shape(b, h, sq, skv, d, workspace_bytes=0).split_parts == 1
-      # a part less than it uses: fewer parts, or none
+      assert (s.workspace_bytes > 0) == (s.split_parts > 1)
+    assert s == shape(b, h, sq, skv, d, workspace_bytes=s.workspace_bytes)
+    none = shape(b, h, sq, skv, d, workspace_bytes=0)
+    assert (none.key_groups, none.split_parts, none.workspace_bytes) == (1, 1, 0)
+    if s.split_parts > 1:
       t = shape(b, h, sq, skv, d, workspace_bytes=s.workspace_bytes - 1)
       assert t.workspace_bytes < s.workspace_bytes
 
@@ -62,15 +63,13 @@ def test_tile_calls_keep_256_row_blocks():
     shape(1, 8, 1024, kv_len=1025)
 
 
-def test_calls_without_a_workspace_argument_have_one_order_of_tiles():
+def test_bad_arguments():
   import ctypes
   lib = _lib.load()
   out, need = (ctypes.c_int32 * 6)(), ctypes.c_size_t(0)
-  for d, sq in ((64, 1024), (128, 512), (128, 8192), (256, 9000)):
-    assert lib.dt_flash_fwd_shape(1, 8, sq, sq, 0, d, _lib.FORM_SINGLE,
-                                  1 << 30, 256, out, ctypes.byref(need)) == 0
-    assert (out[1], out[4], need.value) == (1, 1, 0)
-  for bad in ((1, 8, 64, 64, 0, 128, 3, 0, 256), (1, 8, 64, 64, 0, 128, 0, 0, -1),
+  for bad in ((1, 8, 64, 64, 0, 128, 2, 0, 256), (1, 8, 64, 64, 0, 128, 0, 0, -1),
               (1, 8, 64, 64, 0, 12, 0, 0, 256), (1, 8, 64, 64, 0, 64, 1, 0, 256),
               (0, 8, 64, 64, 0, 128, 0, 0, 256)):
     assert lib.dt_flash_fwd_shape(*bad, out, ctypes.byref(need)) < 0
+  assert lib.dt_flash_fwd_shape(1, 8, 64, 64, 0, 128, 0, 0, 256, None,
+                                ctypes.byref(need)) == _lib.DT_ERR_ARG
