@@ -158,10 +158,11 @@ class AttentionWorkspace:
     if buf is None or buf.numel() < numel:
       buf = torch.empty(numel, device=self.device, dtype=dtype)
       setattr(self, attr, buf)
-      self._views = {}
-    view = self._views.get((attr, numel))
-    if view is None:  # one view per size (slicing costs a microsecond)
-      view = self._views[(attr, numel)] = buf[:numel]
+      self._views.pop(attr, None)
+    view = self._views.get(attr)
+    if view is None or view.numel() != numel:
+      # the last size's view is kept (slicing costs a microsecond)
+      view = self._views[attr] = buf[:numel]
     return view
 
   def packed_v(self, numel):

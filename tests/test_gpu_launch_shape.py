@@ -106,3 +106,13 @@ def test_no_workspace_gives_the_bits_of_the_plain_entry(sp, d, size):
   want = sp.attention(q, k, v)
   assert not torch.equal(want, x)
   assert torch.equal(sp.attention(q, k, v, out=torch.empty_like(q)), want)
+
+
+def test_a_workspace_keeps_one_view_of_each_buffer(sp):
+  banner("workspace views")
+  ws = sp.AttentionWorkspace()
+  for n in (100, 50, 400, 10, 400):
+    view = ws.split(4 * n)
+    assert view.numel() == n and view.data_ptr() == ws._split.data_ptr()
+    assert ws.packed_v(n).numel() == n
+  assert len(ws._views) == 2 and ws._split.numel() == 400
