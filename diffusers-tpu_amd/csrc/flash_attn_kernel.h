@@ -990,9 +990,7 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
   };
 
   // the key loop is unrolled over the ring
-  // (the loop's place within its 64-byte code lines: E4M3 with packed V, B2
-  // H24 S64123 62.0 ms without these 88 bytes, 61.3 with them)
-  if constexpr (QK8 && VT && !SPARSE) asm volatile(".rept 22\n s_nop 0\n .endr");
+  loop_align<!(VT && !QK8)>();
   for (int jt = 0; jt < ntiles; jt += kNStage) {
     iteration(IC<0>{}, jt, sA, sB);
     if (jt + 1 >= ntiles) break;

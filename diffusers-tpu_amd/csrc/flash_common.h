@@ -162,6 +162,22 @@ __device__ __forceinline__ int pack_e4m3x4(uint32_t w0, uint32_t w1) {
                                          true);
 }
 
+// Fixes the place of a key loop's code within 32 bytes, whatever code comes
+// before it: HALF puts the instructions after this 16 bytes past a multiple of
+// 32.  Places 32 bytes apart ran alike, the two halves did not.  First half
+// against second, same process: packed V B1 H40 S48872 37.60 ms, 37.74; E4M3
+// with packed V B2 H24 S64123 60.54, 60.23; row-major H24 S16521 2621 us, 2613;
+// H5 S18900 719.9, 716.5; dim 160 H16 S9000 936.9, 924.9; no difference beyond
+// the noise for E4M3 with row-major V, tile tables and head dims 64, 72 and
+// 256, nor for the shorter calls.
+template <bool HALF>
+__device__ __forceinline__ void loop_align() {
+  if constexpr (HALF)
+    asm volatile(".p2align 5\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0");
+  else
+    asm volatile(".p2align 5");
+}
+
 __device__ __forceinline__ bool wave_any(bool x) {
   return __builtin_amdgcn_ballot_w64(x) != 0;
 }

@@ -627,6 +627,7 @@ __global__ __launch_bounds__(kWNW * 64) void flash_wide_kernel(FlashParams p) {
     kr[i] = kld(WStage<2>{}, i);
     vr[i] = vld(WStage<0>{}, i);
   }
+  loop_align<true>();
   for (int j = 0;; j += 4) {
     iteration(WStage<0>{}, j, sA, sB, pwA, pwB);
     if (j + 1 >= ntiles) break;
