@@ -1200,7 +1200,8 @@ int launch_flash(const FlashParams& base, hipStream_t st) {
   const int grid = p.n_main + p.n_tail * p.n_split;
   hipLaunchKernelGGL((flash_attn_kernel<HD, QK8, SPARSE, VT, R, G>), dim3(grid),
                      dim3(R * G * 64), kLdsBytes, st, p);
-  if (p.n_tail > 0) launch_split_merge<D, BQ>(p, st);
+  if constexpr (R == 8)  // (only whole 256-row blocks are split)
+    if (p.n_tail > 0) launch_split_merge<D, BQ>(p, st);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess)
     return set_error(DT_ERR_LAUNCH, "dt_flash_fwd: %s", hipGetErrorString(e));
