@@ -859,6 +859,22 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
   // ---- prologue: the tiles the iterations before the first would have
   // requested, S(0)
   if constexpr (R == 8) {
+    // a split part other than the first: tile 0 of the whole sweep as well,
+    // its keys only, into the stage that nothing fills before iteration 1
+    if (tbeg > 0) {
+      int kt = 0, rows = kBKV;
+      if constexpr (SPARSE) {
+        kt = __builtin_amdgcn_readfirstlane(tiles[0]);
+        rows = kv_end - kt * kBKV < kBKV ? kv_end - kt * kBKV : kBKV;
+        rows = __builtin_amdgcn_readfirstlane(rows < 0 ? 0 : rows);
+      }
+      const u32x4 rsrc = make_rsrc(
+          (uint64_t)(uintptr_t)kbase + (uint64_t)(kt * kBKV) * krow, rows * krow);
+#pragma unroll
+      for (int i = 0; i < L::kKLoads; ++i)
+        lds_dma16_buf(rsrc, kvo[i],
+                      lds_k + (uint32_t)((kNStage - 1) * L::kKTileB + i * 1024));
+    }
 #pragma unroll
     for (int t = 0; t < kDist; ++t) {
       issue_k(t);
@@ -890,6 +906,41 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
     const int k0 = tile_of(0) * kBKV;
     if (k0 + kBKV > kv_end) mask_tile(sA, k0, hf, kv_end);
   }
+  auto row_max = [&](const f32x16 (&s)[2]) {
+    float mx = s[0][0];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[kb][r]);
+    return fmaxf(mx, __shfl_xor(mx, 32, 64));
+  };
+  // The first tile sets the reference, in its iteration, unless it is set here:
+  // a split part's first tile may lie in masked keys (see kRefGap), where one
+  // sweep would have started from tile 0.  Its row max then stands in.  (Done
+  // here, for such wavefronts alone, the key loop stays the same instructions:
+  // a max handed to the re-base in the loop cost the long sweeps 0.3 to 1.3 %.
+  // A part pays about a tile for it: B2 H24 S4608 414.0 -> 415.7 us.)
+  bool ref_set = fixed;
+  if constexpr (R == 8) {
+    if (tbeg > 0 && !fixed) {
+      phase_a(F{}, IC<kNStage - 1>{}, sB, sB, no_dma);
+      if constexpr (SPARSE) {
+        const int k0 = __builtin_amdgcn_readfirstlane(tiles[0]) * kBKV;
+        if (k0 + kBKV > kv_end) mask_tile(sB, k0, hf, kv_end);
+      }
+      const float mx = row_max(sA), mx0 = row_max(sB);
+      if (wave_any(mx < mx0 - kRefGap)) {
+        ref_set = true;
+        m = (mx < mx0 - kRefGap ? mx0 : mx) - shift;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) negm[r] = -m;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) sA[kb][r] -= m;
+      }
+    }
+  }
   float hsum = softmax_half(sA, 0);
 
   // Key groups: each leaves its row maxes of its first tile behind the rings
@@ -898,12 +949,7 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
   typedef __attribute__((address_space(3))) float lds_f32;
   lds_f32* first_max = (lds_f32*)(lds + G * L::kLds) + wave * 32 + l32;
   if constexpr (G > 1) {
-    float mx = sA[0][0];
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sA[kb][r]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float mx = row_max(sA);
     if (hf == 0) first_max[grp * BQ] = ntiles > 0 ? mx : -INFINITY;
   }
 
@@ -962,7 +1008,7 @@ __global__ __launch_bounds__(R * G * 64, 2) void flash_attn_kernel(FlashParams p
     // instead let the compiler hoist the 16 exps shared by both arms above
     // the branch, out of the MFMA interleave.)
     float sum = hsum + phase_a(T{}, IC<(S + 1) % kNStage>{}, sn, sc, dma);
-    const bool first = jt == 0 && !fixed;
+    const bool first = jt == 0 && !ref_set;
     if (first || wave_any(!(sum <= trip))) {
       float other = -INFINITY;
       if constexpr (G > 1)

@@ -51,10 +51,10 @@ def test_scores_far_below_zero(dta, d, shape):
   assert_attn_close(to64((o / l)[:, h][:, :, rows]), want, "residual")
 
 
-# (B, H, Sq, Skv, D): 4 x 2 and 2 x 4 key groups; split parts above head dim
-# 128 (one sweep each before they were split)
+# (B, H, Sq, Skv, D): 4 x 2 and 2 x 4 key groups; split parts
 MASKED = [(2, 22, 250, 1500, 128), (1, 8, 1000, 1024, 64), (1, 24, 300, 1500, 72),
-          (1, 2, 300, 4096, 256), (1, 3, 200, 2500, 136)]
+          (1, 2, 300, 4096, 256), (1, 3, 200, 2500, 136),
+          (1, 2, 300, 4096, 128), (1, 2, 300, 6000, 64), (1, 2, 300, 4096, 88)]
 
 
 @pytest.mark.parametrize("low", [float("-inf"), torch.finfo(torch.bfloat16).min])
@@ -66,7 +66,7 @@ def test_masked_tiles_after_the_first(dta, case, low):
   banner(f"masked tiles {case} {low}")
   if torch.cuda.get_device_properties(0).multi_processor_count == 256:
     s = launch_shape(b, h, sq, skv, d)
-    assert s.key_groups > 1 if d <= 128 else s.split_parts > 1
+    assert s.key_groups > 1 or s.split_parts > 1
   q, k, v = _inputs(b, h, sq, skv, d, 660)
   q[..., 0], k[..., 0] = 1.0, 0.0
   keep = np.r_[0:64, skv - 5:skv]
@@ -77,3 +77,23 @@ def test_masked_tiles_after_the_first(dta, case, low):
   assert_attn_close(to64(got[:1, :2]), want, "masked")
   o, m, l = dta.residual_attention(q, k, v)
   assert_attn_close(to64((o / l)[:1, :2]), want, "residual")
+
+
+@pytest.mark.parametrize("low", [float("-inf"), torch.finfo(torch.bfloat16).min])
+@pytest.mark.parametrize("skv", [4000, 4096])
+def test_masked_tiles_of_a_table(dta, skv, low):
+  """Split parts of a tile table's sweep, whose first tile is any tile (the
+  second query block lists only the last, partial one)."""
+  from diffusers_tpu_amd.kernels import sparse_splash
+  banner(f"masked tiles of a table, {skv} {low}")
+  q, k, v = _inputs(1, 2, 500, skv, 128, 670)
+  q[..., 0], k[..., 0] = 1.0, 0.0
+  tiles = -(-skv // 64)
+  rows = [[0] + list(range(2, tiles)), [tiles - 1]]
+  k[:, :, 64:skv - 5, 0] = low
+  got = sparse_splash.attention(q, k, v, block_q=256, block_kv=64, kv_table=rows)
+  for lo, hi, keep in ((0, 256, np.r_[0:64, skv - 5:skv]),
+                       (256, 500, np.r_[skv - 5:skv])):
+    want = A.attention_f64(to64(q[:, :, lo:hi]), to64(k[:, :, keep]),
+                           to64(v[:, :, keep]))
+    assert_attn_close(to64(got[:, :, lo:hi]), want, f"rows {lo}:{hi}")
