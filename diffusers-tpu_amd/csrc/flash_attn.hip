@@ -12,8 +12,12 @@ SplitPlan split_plan(int64_t n_wg, int ntiles, int n_cu, int D, int bq,
   const int64_t rem = n_wg % n_cu;
   if (rem == 0) return sp;
   // Short sweeps over many rounds: the idle CUs of the last one are a few
-  // percent of the call at most, about what the split's second launch costs
-  // (H40 Sq 48360, 8 tiles, 29.8 rounds: 610 us with it, 606 without).
+  // percent of the call at most, and the split's second launch costs as much.
+  // (It decides for E4M3 keys, tile tables and dims above 128: bf16 calls of so
+  // few tiles run 128-row workgroups.)  E4M3, H40 Sq 15000, 9.2 rounds, whole
+  // against split, us: 8 tiles 164.3, 169.5 in 2; 12 tiles 217.1, 217.0 in 3; 16
+  // tiles 265.4, 270.8 in 4; past the line 17 tiles 282.0, 283.2, 24 tiles
+  // 367.6, 370.1.  At 4.9 to 29.5 rounds of other fillings nothing would split.
   if (ntiles <= 16 && n_wg >= 8 * (int64_t)n_cu) return sp;
   // The last round's rem query blocks cut into ns parts run as
   // ceil(rem * ns / n_cu) rounds of parts of ntiles / ns tiles; each
@@ -103,6 +107,12 @@ int device_cu_count(int* n_cu) {
 // 33.6 -> 29.6, H96 S1024 70.1 -> 57.5; kept 8 x 1: H2 S4096 (split 10 ways)
 // 33.8 against 49.5, H24 S2048 52.4 against 57.6.  D = 64: H8 S1024
 // 16.3 -> 10.6, H16 S2048 29.7 -> 24.6, kept H8 S4096 44.9 against 47.0.
+// Dims in between take the constants of their width, D = 64 or 128.  All
+// shapes forced at 15 sizes around the lines (2 to 48 heads, 512 to 4096 rows),
+// the chosen against the fastest: D = 128 0.2 % slower on average and 2.2 % at
+// most, 104 0.2 and 2.1, 72 1.2 and 5.9 (H8 S1024: 17.3 us in 4 x 1, 16.3 in 4
+// x 2), 64 0.1 and 0.9, 40 0.3 and 4.8 (B2 H24 S700: 16.1 in 4 x 1, 15.4 in 8 x
+// 1).
 struct RowShape {
   int r, g;
 };
