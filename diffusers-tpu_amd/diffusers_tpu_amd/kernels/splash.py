@@ -174,11 +174,11 @@ class AttentionWorkspace:
     return self._get("_split", (nbytes + 3) // 4, torch.float32)
 
   def reserve(self, query_shape, key_shape, kv_len=None, *, packed=None):
-    """Allocates what a call with these shapes needs in any form (``kv_len``
-    an int or ``None``; a device length plans for every key): the split of
-    256-row blocks, also where the bf16 call runs in smaller workgroups and
-    leaves it to calls with ``qk_fp8``.  ``packed``: whether the call streams
-    packed V (default: as ``attention`` decides)."""
+    """Allocates what a call with these shapes needs (``kv_len`` an int or
+    ``None``; a device length plans for every key): the split of 256-row
+    blocks at the kernel's width, also where the bf16 call runs in smaller
+    workgroups and leaves it to a call with ``qk_fp8``.  ``packed``: whether
+    the call streams packed V (default: as ``attention`` decides)."""
     b, hq, sq, d = query_shape
     _, hkv, skv, _ = key_shape
     # a device length, or per-sample lengths: plan for every key

@@ -14,7 +14,7 @@ SHAPES = [
     # (B, Hq, Hkv, Sq, Skv, kv_len)
     (1, 1, 1, 1, 1, None),
     (2, 4, 2, 129, 200, 131),
-    (1, 2, 2, 300, 4096, None),     # split parts
+    (1, 2, 2, 300, 4096, None),     # split parts (key groups up to 64)
     (1, 3, 3, 4200, 130, None),     # many row blocks, a short sweep
 ]
 

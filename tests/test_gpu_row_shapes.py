@@ -2,7 +2,8 @@
 run in 128- or 64-row workgroups, with the tiles dealt to key groups of one
 workgroup.  Sizes at the edges of the row blocks (64, 128, 256 rows), of the
 tiles (64 keys) and of the groups (fewer tiles than groups), against the
-float64 oracle."""
+float64 oracle.  (Which shape each size runs in, and lengths that leave a
+group without tiles: test_gpu_launch_shape.)"""
 import numpy as np
 import pytest
 import torch
@@ -17,7 +18,7 @@ CASES = [(b, hq, hkv, sq, skv, n, d)
          for d in (64, 128)
          for b, hq, hkv, sq, skv, n in [
              (1, 1, 1, 1, 1, None),            # one row, one key
-             (1, 2, 2, 65, 64, None),          # one tile: groups without any
+             (1, 2, 2, 65, 64, None),          # one tile
              (2, 2, 1, 129, 300, (65, 0)),     # device lengths, one of them 0
              (1, 3, 3, 128, 1087, None),       # 17 tiles, the last of 63 keys
              (2, 4, 2, 255, 1300, (1281, 1)),  # 21 tiles against 1
