@@ -65,7 +65,7 @@ def test_shape_matches_oracle(sp, d, want, size):
 @pytest.mark.parametrize("d", [64, 128])
 def test_smaller_workgroups_take_no_workspace(sp, d):
   """Calls that run in smaller workgroups hold no split buffer; reserve still
-  covers every form of a call of the shape."""
+  sizes the one that an E4M3 call of the shape uses."""
   banner(f"workspace of small shapes, dim {d}")
   q = seeded((1, 8, 500, d), 710)
   ws = sp.AttentionWorkspace()
